@@ -342,14 +342,15 @@ struct GemmStage {
 // device copy of the block-form MPO-term sum; the FP32 coefficient table is made on first use
 struct SAsmStage {
     SBlock* blocks = nullptr;
-    SWork* work = nullptr;
+    SWork *work = nullptr, *launch = nullptr;
     int64_t* utile = nullptr;
     uint32_t* kstep = nullptr;
     double* ualpha = nullptr;
     float* ualpha32 = nullptr;
     int64_t* lsoff = nullptr;
     int32_t* llds = nullptr;
-    int64_t n_work = 0;
+    SWorkCounts n_work;
+    int64_t n_launch = 0;
     uint64_t n_alpha = 0;
     // small-tile lines
     SSmallWork* swork = nullptr;
@@ -366,7 +367,9 @@ struct SAsmStage {
         ualpha = dev_upload(B.ualpha, s);
         lsoff = dev_upload(B.lsoff, s);
         llds = dev_upload(B.llds, s);
-        n_work = int64_t(B.work.size());
+        launch = dev_upload(B.launch, s);
+        n_launch = int64_t(B.launch.size());
+        n_work = B.n_work;
         n_alpha = B.ualpha.size();
         swork = dev_upload(B.small_work, s);
         slines = dev_upload(B.small_lines, s);
@@ -374,8 +377,8 @@ struct SAsmStage {
         n_swork = int64_t(B.small_work.size());
     }
     void run(const double* T, double* S, hipStream_t s) const {
-        if (n_work)
-            hipcheck(launch_sblocks<double>(blocks, work, n_work, utile, kstep, ualpha, lsoff, llds, T, S, xcd_contiguous, s),
+        if (n_launch)
+            hipcheck(launch_sblocks<double>(blocks, launch, n_launch, work, n_work, utile, kstep, ualpha, lsoff, llds, T, S, xcd_contiguous, s),
                      "S-assembly");
         if (n_swork) hipcheck(launch_small_lines<double>(swork, n_swork, slines, sterms, T, S, s), "S-assembly");
     }
@@ -387,19 +390,20 @@ struct SAsmStage {
     }
     void run32(const float* T, float* S, hipStream_t s) {
         ensure32(s);
-        if (n_work)
-            hipcheck(launch_sblocks<float>(blocks, work, n_work, utile, kstep, ualpha32, lsoff, llds, T, S, xcd_contiguous,
+        if (n_launch)
+            hipcheck(launch_sblocks<float>(blocks, launch, n_launch, work, n_work, utile, kstep, ualpha32, lsoff, llds, T, S, xcd_contiguous,
                                            s),
                      "S-assembly");
         if (n_swork) hipcheck(launch_small_lines<float>(swork, n_swork, slines, sterms, T, S, s), "S-assembly");
     }
     void release() {
-        dev_free(blocks); dev_free(work); dev_free(utile); dev_free(kstep); dev_free(ualpha); dev_free(ualpha32);
+        dev_free(blocks); dev_free(work); dev_free(launch); dev_free(utile); dev_free(kstep); dev_free(ualpha); dev_free(ualpha32);
         dev_free(lsoff); dev_free(llds); dev_free(swork); dev_free(slines); dev_free(sterms);
-        blocks = nullptr; work = nullptr; utile = nullptr; kstep = nullptr; ualpha = nullptr; ualpha32 = nullptr;
+        blocks = nullptr; work = launch = nullptr; utile = nullptr; kstep = nullptr; ualpha = nullptr; ualpha32 = nullptr;
         lsoff = nullptr;
         llds = nullptr; swork = nullptr; slines = nullptr; sterms = nullptr;
-        n_work = 0;
+        n_work = SWorkCounts();
+        n_launch = 0;
         n_swork = 0;
     }
 };
@@ -843,7 +847,7 @@ static void run_growth(mq_ctx_t ctx, GrowPlanHost& P, double const* bnd, double 
     nb->n = P.out_elems;
     nb->data = dev_alloc<double>(nb->n);
     nb->hold = own_device(nb->data);
-    double* T = dev_alloc<double>(P.t_elems);
+    double* T = dev_alloc<double>(P.t_elems + SB_T_SPARE);
     double* S = dev_alloc<double>(P.s_elems);
     GemmStage tg, cg;
     SAsmStage sa;
@@ -1079,7 +1083,7 @@ static void finish_plan(mq_ctx_t ctx, mq_hpsi_plan_s* p, std::vector<LpanelPart>
                         uint64_t(j.dst) + uint64_t(j.rows) * j.cols * j.nblocks <= H.lpanel_elems,
                     "L panel job outside its buffers");
     p->r_elems = r_n;
-    p->T = dev_alloc<double>(H.t_buf);
+    p->T = dev_alloc<double>(H.t_buf + SB_T_SPARE);
     p->S = dev_alloc<double>(H.s_buf);
     p->Lpanel = dev_alloc<double>(H.lpanel_elems);
     p->gemm_ws = dev_alloc<double>(ws_max);

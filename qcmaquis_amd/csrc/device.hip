@@ -262,163 +262,185 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmDesc* __rest
     }
 }
 
-// Block-form MPO-term sum on the matrix cores.  A work item is SBLOCK_ELEMS consecutive tile
-// elements of one block of up to SBLOCK_GROUPS groups of 16 lines; each of the SB_WAVES waves owns
-// 16 * SB_NC of them.  Per k-step (4 union tiles) every group that reads one of its tiles computes
-// Y_g(16 lines x 16 elements) += alpha_g(16 x 4) * X(4 tiles x 16 elements) on the matrix cores:
-// lane l loads element l % 16 of tile l / 16 (16 consecutive values per tile, shared by the
-// groups) and alpha of line l % 16 for tile l / 16.  The tile offsets, k-step words and
-// coefficient sub-blocks are staged in LDS, SB_KCHUNK k-steps at a time; the next chunk's tables
-// are loaded into registers while the current chunk is summed, and the tiles of the next
-// SB_UNROLL k-steps are loaded while the current ones go through the matrix cores.  The k-step's
-// group mask is read into a scalar register, so the groups without a sub-block are skipped by the
-// whole wave.
-#ifndef MQ_SB_NC
-#define MQ_SB_NC 2
-#endif
-#ifndef MQ_SB_UNROLL
-#define MQ_SB_UNROLL 2
-#endif
-#ifndef MQ_SB_KCHUNK
-#define MQ_SB_KCHUNK 8
-#endif
-#ifndef MQ_SB_WAVES_PER_EU
-#define MQ_SB_WAVES_PER_EU 4
-#endif
-constexpr int SB_NC = MQ_SB_NC;                         // 16-element column tiles per wave
+// Block-form MPO-term sum on the matrix cores.  Per k-step (4 union tiles) every group of 16 lines
+// that reads one of its tiles computes Y_g(16 lines x 16 elements) += alpha_g(16 x 4) * X(4 tiles x
+// 16 elements): lane l supplies element l % 16 of tile l / 16 and alpha of line l % 16 for tile
+// l / 16.  A wave owns 32 tile elements: lane l loads the consecutive elements 2 (l % 16) and
+// 2 (l % 16) + 1 of its tile in one access, column tile j of the matrix-core steps takes the
+// elements of parity j, and the lane's results are consecutive elements of S again.  Coefficients and
+// tile offsets go to LDS without passing through registers.  The waves of a workgroup work by the
+// block's tile size (SWorkCounts): one block on all of them (SBLOCK_ELEMS elements, tables staged
+// once per workgroup), a block of 33 to 64 elements on two, or one block per wave; in the last two
+// every wave stages its own block's tables and runs without barriers.
+//
+// Bound: L2-miss traffic (every block reads the union of its T tiles, T 2.1-2.5 times in all, and
+// writes S) where tiles are large, waiting on the chain tables -> tiles -> matrix cores where they
+// are small.  Staging a whole block's tables at once (most blocks fit one pass) in place of eight
+// k-steps at a time behind two barriers each, one 16-byte load per k-step instead of two of 8, and
+// line tables read once through LDS cut the vector-memory instructions to a third.  FP64, before ->
+// now: 18 orbitals, TwoU1, M = 509 1.64 -> 0.81 ms; 20 orbitals, SU2U1, M = 700 2.82 -> 1.80 ms,
+// M = 2048 19.2 -> 14.1 ms (75 GB read and written); FP32 there 10.97 -> 8.02 ms.  Without barriers
+// at all (every wave its own loads into registers) the first took 1.36 ms; four column tiles per
+// wave 1.02 ms; two or four k-steps of loads in flight 0.93 and 0.95 where three took 0.92.
 constexpr int SB_XCDS = 8;                              // XCDs of an MI355X
-constexpr int SB_WAVES = SBLOCK_ELEMS / (16 * SB_NC);   // waves per workgroup
+constexpr int SB_SUB = 64;                              // coefficient sub-blocks staged per workgroup
+constexpr int SB_KS = 64;                               // k-steps staged per workgroup
+constexpr int SB_NC = 2;                                // column tiles per wave
+constexpr int SB_U = 3;                                 // k-steps whose tile loads are issued together
 constexpr int SB_THREADS = 64 * SB_WAVES;
-constexpr int SB_UNROLL = MQ_SB_UNROLL;                 // k-steps whose loads are issued together
-constexpr int SB_KCHUNK = MQ_SB_KCHUNK;                 // k-steps staged in LDS at a time
-constexpr int SB_ST_ALPHA = SB_KCHUNK * SBLOCK_GROUPS * 64 / SB_THREADS;  // staged values per thread
-static_assert(SBLOCK_GROUP == 16 && SB_WAVES * 16 * SB_NC == SBLOCK_ELEMS && SB_WAVES <= 16, "S block geometry");
-static_assert(SB_KCHUNK % (2 * SB_UNROLL) == 0, "staged chunks hold whole double-buffered k-step groups");
-static_assert(4 * SB_KCHUNK <= SB_THREADS && SB_ST_ALPHA * SB_THREADS == SB_KCHUNK * SBLOCK_GROUPS * 64,
-              "one staging pass covers a chunk's tables");
+constexpr int SB_SUB1 = SB_SUB / SB_WAVES, SB_KS1 = SB_KS / SB_WAVES;  // one wave's share of the staging
+static_assert(SBLOCK_GROUP == 16 && 16 * SB_NC == 32 && SB_WAVES * 16 * SB_NC == SBLOCK_ELEMS && SB_WAVES % 2 == 0 && SB_SUB1 >= SBLOCK_GROUPS && SB_KS <= 64,
+              "S block geometry");
+
+// n bytes (a multiple of 16) from src to LDS at dst (both 16-byte aligned) by `lanes` lanes of whole
+// waves, this one being number `lane`; in flight until the wave's next wait for vector memory
+__device__ inline void lds_fetch(const void* src, void* dst, int n, int lane, int lanes) {
+    const char* s = static_cast<const char*>(src);
+    char* d = static_cast<char*>(dst);
+    for (int o = __builtin_amdgcn_readfirstlane(lane & ~63) * 16; o < n; o += lanes * 16)
+        if (o + 16 * (lane & 63) < n)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(s + o + 16 * (lane & 63)),
+                                             (__attribute__((address_space(3))) void*)(d + o), 16, 0, 0);
+}
+
+// two consecutive elements at any element alignment
+template <class T> struct PairOf { typedef T type __attribute__((ext_vector_type(2), aligned(sizeof(T)))); };
 
 template <class T>
-__global__ __launch_bounds__(SB_THREADS) __attribute__((amdgpu_waves_per_eu(MQ_SB_WAVES_PER_EU))) void sblock_kernel(const SBlock* __restrict__ blocks, const SWork* __restrict__ work,
-                                                     const int64_t* __restrict__ utile, const uint32_t* __restrict__ kstep,
-                                                     const T* __restrict__ ualpha, const int64_t* __restrict__ lsoff,
-                                                     const int32_t* __restrict__ llds, const T* __restrict__ X,
-                                                     T* __restrict__ S, int xcd_contiguous) {
+__global__ __launch_bounds__(SB_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void sblock_kernel(
+    const SBlock* __restrict__ blocks, const SWork* __restrict__ launch, const SWork* __restrict__ work, SWorkCounts n,
+    const int64_t* __restrict__ utile, const uint32_t* __restrict__ kstep, const T* __restrict__ ualpha,
+    const int64_t* __restrict__ lsoff, const int32_t* __restrict__ llds, const T* __restrict__ X, T* __restrict__ S,
+    int xcd_contiguous) {
     typedef typename Mma<T>::acc_t acc_t;
-    __shared__ int64_t uts[4 * SB_KCHUNK];
-    __shared__ uint32_t kws[SB_KCHUNK];
-    __shared__ T uas[SB_KCHUNK * SBLOCK_GROUPS * 64];
+    typedef typename PairOf<T>::type pair_t;
+    __shared__ __attribute__((aligned(16))) T s_alpha[SB_SUB * 64];
+    __shared__ __attribute__((aligned(16))) int64_t s_off[SB_KS * 4];
+    __shared__ __attribute__((aligned(16))) int64_t s_lsoff[SB_WAVES * SBLOCK_LINES];
+    __shared__ __attribute__((aligned(16))) int32_t s_llds[SB_WAVES * SBLOCK_LINES];
     // Workgroups are dispatched to the XCDs in turn (workgroup i on XCD i mod 8); with
     // xcd_contiguous each XCD takes a contiguous range of the work list instead, so consecutive
     // work items (neighbouring blocks' slices of shared T tiles) meet in one XCD's L2.  The map is
     // a bijection of [0, gridDim.x).
-    int64_t wi = blockIdx.x;
+    int wg = int(blockIdx.x);
     if (xcd_contiguous) {
-        const int64_t n = gridDim.x, q = n / SB_XCDS, r = n % SB_XCDS;
-        const int64_t x = blockIdx.x % SB_XCDS, k = blockIdx.x / SB_XCDS;
-        wi = x < r ? x * (q + 1) + k : r * (q + 1) + (x - r) * q + k;
+        const int nw = int(gridDim.x), q = nw / SB_XCDS, r = nw % SB_XCDS;
+        const int x = wg % SB_XCDS, k = wg / SB_XCDS;
+        wg = x < r ? x * (q + 1) + k : r * (q + 1) + (x - r) * q + k;
     }
-    const SWork w = work[wi];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    SWork w = launch[wg];
+    const bool team = w.blk >= 0;
+    int sub = wave;  // this wave's slice of its work item
+    if (!team) {     // -w.blk waves per item, from work[w.n0]
+        const int lw = -w.blk - 1, wi = w.n0 + (wave >> lw);
+        sub = wave & lw;
+        if (wi >= (lw ? n.team + n.pair : n.team + n.pair + n.solo)) return;
+        w = work[wi];
+    }
     const SBlock b = blocks[w.blk];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n0 = w.n0 + wave * 16 * SB_NC;
-    // a wave past the tile end loads and stores nothing but takes part in the barriers
+    const int n0 = w.n0 + 16 * SB_NC * sub;
+    // a wave past the tile end loads and stores no tile but takes part in its team's barriers
     const bool active = n0 < b.E;
+    if (!team && !active) return;
     const int li = lane & 15, lk = lane >> 4;
+    T* al = s_alpha + (team ? 0 : wave * SB_SUB1 * 64);
+    int64_t* of = s_off + (team ? 0 : wave * SB_KS1 * 4);
+    int64_t* so = s_lsoff + (team ? 0 : wave * SBLOCK_LINES);
+    int32_t* ld = s_llds + (team ? 0 : wave * SBLOCK_LINES);
+    const int cap_sub = team ? SB_SUB : SB_SUB1, cap_k = team ? SB_KS : SB_KS1;
+    const int st_lane = team ? int(threadIdx.x) : lane, st_lanes = team ? SB_THREADS : 64;
+    const uint32_t* kw = kstep + b.k_off;
+    // this lane's elements e0, e0 + 1; past the tile's end it reads what follows the tile in
+    // the T buffer (SB_T_SPARE elements after the last one) and stores none of it
+    const int e0 = n0 + 2 * li;
+    const int ec = e0 < b.E ? e0 : b.E - 1;
     acc_t acc[SBLOCK_GROUPS][SB_NC];
 #pragma unroll
     for (int g = 0; g < SBLOCK_GROUPS; ++g)
 #pragma unroll
         for (int j = 0; j < SB_NC; ++j) acc[g][j] = acc_t{0, 0, 0, 0};
-    const int64_t* ut = utile + 4 * int64_t(b.k_off);
-    const uint32_t* kw = kstep + b.k_off;
-    const T* ua = ualpha + 64 * b.a_off;
 
-    // the tables of the chunk from k-step c0 in registers: this thread's slot offset, k-step word
-    // and coefficient values; ra0 / ra1 = the chunk's sub-block range
-    int64_t r_ut = -1;
-    uint32_t r_kw = 0;
-    T r_a[SB_ST_ALPHA];
-    int ra0 = 0, ra1 = 0;
-    auto fetch = [&](int c0) {
-        const int cn = b.nk - c0 < SB_KCHUNK ? b.nk - c0 : SB_KCHUNK;
-        ra0 = int(kw[c0] >> 8);
-        ra1 = c0 + cn < b.nk ? int(kw[c0 + cn] >> 8) : b.na;
-        if (tid < 4 * cn) r_ut = ut[4 * c0 + tid];
-        if (tid < cn) r_kw = kw[c0 + tid];
+    lds_fetch(lsoff + b.line0, so, SBLOCK_LINES * 8, st_lane, st_lanes);
+    lds_fetch(llds + b.line0, ld, SBLOCK_LINES * 4, st_lane, st_lanes);
+    for (int c0 = 0; c0 < b.nk;) {
+        // the next k-steps whose tables fit: lane l looks at k-step c0 + l
+        const int kl = c0 + lane;
+        const uint32_t word = kl < b.nk ? kw[kl] : 0;
+        const int a0 = __builtin_amdgcn_readfirstlane(int(word >> 8));
+        const int end = kl + 1 < b.nk ? int(kw[kl + 1] >> 8) : b.na;
+        const int cn = __builtin_popcountll(__ballot(kl < b.nk && lane < cap_k && end - a0 <= cap_sub));
+        const int an = __builtin_amdgcn_readlane(end, cn - 1) - a0;
+        if (team && c0 > 0) __syncthreads();  // the previous k-steps' tables are consumed
+        asm volatile("" ::: "memory");
+        lds_fetch(utile + 4 * (int64_t(b.k_off) + c0), of, 32 * cn, st_lane, st_lanes);
+        lds_fetch(ualpha + 64 * (b.a_off + a0), al, 64 * int(sizeof(T)) * an, st_lane, st_lanes);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (team) __syncthreads();
+        if (active) {
+            // the tile elements of the k-steps [k, k + SB_U)
+            auto load_x = [&](pair_t (&x)[SB_U], int k) {
 #pragma unroll
-        for (int q = 0; q < SB_ST_ALPHA; ++q) {
-            const int i = tid + SB_THREADS * q;
-            r_a[q] = i < 64 * (ra1 - ra0) ? ua[64 * int64_t(ra0) + i] : T(0);
-        }
-    };
-    // X of the k-steps [k, k + SB_UNROLL) of the staged chunk (cn k-steps)
-    auto load_x = [&](T (&x)[SB_UNROLL][SB_NC], int k, int cn) {
+                for (int u = 0; u < SB_U; ++u) {
+                    const int64_t o = k + u < cn ? of[4 * (k + u) + lk] : -1;
+                    const pair_t v = *reinterpret_cast<const pair_t*>(X + (o < 0 ? 0 : o) + ec);
 #pragma unroll
-        for (int u = 0; u < SB_UNROLL; ++u) {
-            const int64_t to = k + u < cn ? uts[4 * (k + u) + lk] : -1;
+                    for (int j = 0; j < SB_NC; ++j) x[u][j] = o < 0 ? T(0) : v[j];  // empty slot (last k-step): a zero tile
+                }
+            };
+            auto mma = [&](pair_t (&x)[SB_U], int k) {
 #pragma unroll
-            for (int j = 0; j < SB_NC; ++j) {
-                const int e = n0 + 16 * j + li;
-                x[u][j] = (to >= 0 && e < b.E) ? X[to + e] : T(0);  // B[tile lk][element e]
+                for (int u = 0; u < SB_U; ++u) {
+                    if (k + u >= cn) break;
+                    const uint32_t wd = __builtin_amdgcn_readlane(word, k + u);
+                    const T* pa = al + 64 * (int(wd >> 8) - a0) + lane;
+#pragma unroll
+                    for (int g = 0; g < SBLOCK_GROUPS; ++g)
+                        if ((wd >> g) & 1u) {
+                            const T a = *pa;
+                            pa += 64;
+#pragma unroll
+                            for (int j = 0; j < SB_NC; ++j) acc[g][j] = Mma<T>::step(a, x[u][j], acc[g][j]);
+                        }
+                }
+            };
+            pair_t xa[SB_U], xb[SB_U];
+            load_x(xa, 0);
+            for (int k = 0; k < cn; k += 2 * SB_U) {
+                load_x(xb, k + SB_U);
+                mma(xa, k);
+                load_x(xa, k + 2 * SB_U);
+                mma(xb, k + SB_U);
             }
         }
-    };
-    auto mma = [&](T (&x)[SB_UNROLL][SB_NC], int k, int cn, int a0) {
-#pragma unroll
-        for (int u = 0; u < SB_UNROLL; ++u) {
-            if (k + u >= cn) break;
-            const uint32_t word = __builtin_amdgcn_readfirstlane(kws[k + u]);
-            int ai = int(word >> 8) - a0;
-#pragma unroll
-            for (int g = 0; g < SBLOCK_GROUPS; ++g) {
-                if (!((word >> g) & 1u)) continue;
-                const T a = uas[64 * ai + lane];  // A[line li][tile lk]
-                ++ai;
-#pragma unroll
-                for (int j = 0; j < SB_NC; ++j) acc[g][j] = Mma<T>::step(a, x[u][j], acc[g][j]);
-            }
-        }
-    };
-
-    if (b.nk > 0) fetch(0);
-    for (int c0 = 0; c0 < b.nk; c0 += SB_KCHUNK) {
-        const int cn = b.nk - c0 < SB_KCHUNK ? b.nk - c0 : SB_KCHUNK;
-        const int a0 = ra0;
-        __syncthreads();  // the previous chunk's tables are consumed
-        if (tid < 4 * cn) uts[tid] = r_ut;
-        if (tid < cn) kws[tid] = r_kw;
-#pragma unroll
-        for (int q = 0; q < SB_ST_ALPHA; ++q) {
-            const int i = tid + SB_THREADS * q;
-            if (i < 64 * (ra1 - ra0)) uas[i] = r_a[q];
-        }
-        __syncthreads();
-        if (c0 + SB_KCHUNK < b.nk) fetch(c0 + SB_KCHUNK);
-        if (!active) continue;
-        T xa[SB_UNROLL][SB_NC], xb[SB_UNROLL][SB_NC];
-        load_x(xa, 0, cn);
-        for (int ks = 0; ks < cn; ks += 2 * SB_UNROLL) {
-            load_x(xb, ks + SB_UNROLL, cn);
-            mma(xa, ks, cn, a0);
-            load_x(xa, ks + 2 * SB_UNROLL, cn);
-            mma(xb, ks + SB_UNROLL, cn, a0);
-        }
+        c0 += cn;
     }
-    if (!active) return;
-    // register r of lane l holds Y_g[line row(l, r)][element l % 16]
-#pragma unroll
-    for (int j = 0; j < SB_NC; ++j) {
-        const int e = n0 + 16 * j + li;
-        if (e >= b.E) continue;
-        const int r_ = e % b.rows, c_ = e / b.rows;
-#pragma unroll
-        for (int g = 0; g < SBLOCK_GROUPS; ++g)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int i = SBLOCK_GROUP * g + Mma<T>::row(lane, r);
-                if (i < b.nlines) S[lsoff[b.line0 + i] + r_ + int64_t(c_) * llds[b.line0 + i]] = acc[g][j][r];
-            }
+    if (b.nk == 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (team) __syncthreads();
     }
+    if (!active || e0 >= b.E) return;
+    // register r of lane l holds Y_g[line row(l, r)][element]: the lane's elements are stored at once
+    // unless a tile column ends among them
+    const int r_ = e0 % b.rows, c_ = e0 / b.rows;
+    const bool whole = r_ + 1 < b.rows;
+#pragma unroll
+    for (int g = 0; g < SBLOCK_GROUPS; ++g)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int i = SBLOCK_GROUP * g + Mma<T>::row(lane, r);
+            if (i >= b.nlines) continue;
+            T* p = S + so[i] + r_ + int64_t(c_) * ld[i];
+            if (whole) {
+                pair_t v;
+                v.x = acc[g][0][r];
+                v.y = acc[g][1][r];
+                *reinterpret_cast<pair_t*>(p) = v;
+            } else {
+                *p = acc[g][0][r];
+                if (e0 + 1 < b.E) p[int64_t(ld[i]) - r_] = acc[g][1][r];
+            }
+        }
 }
 
 // Small-tile MPO-term sum: a work item is up to 256 >> lg lines of 2^lg lanes each (tile elements
@@ -702,22 +724,21 @@ hipError_t launch_slines(const SLine* lines, int64_t n_lines, const STerm* terms
 }
 
 template <class T>
-hipError_t launch_sblocks(const SBlock* blocks, const SWork* work, int64_t n_work, const int64_t* utile,
-                          const uint32_t* kstep, const T* ualpha, const int64_t* lsoff, const int32_t* llds,
-                          const T* X, T* S, bool xcd_contiguous, hipStream_t stream) {
-    for (int64_t off = 0; off < n_work; off += 0x7fffffff) {
-        int64_t cnt = n_work - off < 0x7fffffff ? n_work - off : 0x7fffffff;
-        hipLaunchKernelGGL(sblock_kernel<T>, dim3(unsigned(cnt)), dim3(SB_THREADS), 0, stream, blocks, work + off, utile,
-                           kstep, ualpha, lsoff, llds, X, S, int(xcd_contiguous));
-    }
+hipError_t launch_sblocks(const SBlock* blocks, const SWork* launch, int64_t n_launch, const SWork* work, SWorkCounts n,
+                          const int64_t* utile, const uint32_t* kstep, const T* ualpha, const int64_t* lsoff,
+                          const int32_t* llds, const T* X, T* S, bool xcd_contiguous, hipStream_t stream) {
+    if (n_launch > 0x7fffffff) return hipErrorInvalidValue;
+    if (n_launch > 0)
+        hipLaunchKernelGGL(sblock_kernel<T>, dim3(unsigned(n_launch)), dim3(SB_THREADS), 0, stream, blocks, launch, work, n,
+                           utile, kstep, ualpha, lsoff, llds, X, S, int(xcd_contiguous));
     return hipGetLastError();
 }
-template hipError_t launch_sblocks<double>(const SBlock*, const SWork*, int64_t, const int64_t*, const uint32_t*,
-                                           const double*, const int64_t*, const int32_t*, const double*, double*, bool,
-                                           hipStream_t);
-template hipError_t launch_sblocks<float>(const SBlock*, const SWork*, int64_t, const int64_t*, const uint32_t*,
-                                          const float*, const int64_t*, const int32_t*, const float*, float*, bool,
-                                          hipStream_t);
+template hipError_t launch_sblocks<double>(const SBlock*, const SWork*, int64_t, const SWork*, SWorkCounts,
+                                           const int64_t*, const uint32_t*, const double*, const int64_t*,
+                                           const int32_t*, const double*, double*, bool, hipStream_t);
+template hipError_t launch_sblocks<float>(const SBlock*, const SWork*, int64_t, const SWork*, SWorkCounts,
+                                          const int64_t*, const uint32_t*, const float*, const int64_t*, const int32_t*,
+                                          const float*, float*, bool, hipStream_t);
 
 template <class T>
 hipError_t launch_small_lines(const SSmallWork* work, int64_t n_work, const SLine* lines, const STerm* terms,

@@ -30,9 +30,9 @@ hipError_t launch_gemm(GemmPrec prec, const GemmDesc* probs, const GemmRow* rows
 // block-form MPO-term sum (SBlockTable uploaded; alpha, T and S of type T): writes every S tile
 // of the table's lines; xcd_contiguous: each XCD takes a contiguous range of the work list
 template <class T>
-hipError_t launch_sblocks(const SBlock* blocks, const SWork* work, int64_t n_work, const int64_t* utile,
-                          const uint32_t* kstep, const T* ualpha, const int64_t* lsoff, const int32_t* llds,
-                          const T* X, T* S, bool xcd_contiguous, hipStream_t stream);
+hipError_t launch_sblocks(const SBlock* blocks, const SWork* launch, int64_t n_launch, const SWork* work, SWorkCounts n,
+                          const int64_t* utile, const uint32_t* kstep, const T* ualpha, const int64_t* lsoff,
+                          const int32_t* llds, const T* X, T* S, bool xcd_contiguous, hipStream_t stream);
 // small-tile MPO-term sum (SBlockTable small_* tables uploaded; T and S of type T, coefficients
 // FP64, rounded to T): writes the S tiles of the small lines
 template <class T>

@@ -1594,16 +1594,52 @@ SBlockTable build_sblocks(HostTable<SLine> const& lines, HostTable<STerm> const&
     }
     // work items: block by block, or (panel > 0) per panel of up to `panel` consecutive blocks of
     // one tile shape, element range by element range, so that neighbouring blocks -- which share
-    // most of their union tiles -- read the same slice of those tiles in consecutive items
-    for (int32_t p0 = 0; p0 < int32_t(nb);) {
-        int32_t p1 = p0 + 1;
-        if (panel > 0)
-            while (p1 < int32_t(nb) && p1 - p0 < panel && B.blocks[size_t(p1)].E == B.blocks[size_t(p0)].E &&
-                   B.blocks[size_t(p1)].rows == B.blocks[size_t(p0)].rows)
-                ++p1;
-        for (int32_t e = 0; e < B.blocks[size_t(p0)].E; e += SBLOCK_ELEMS)
-            for (int32_t bi = p0; bi < p1; ++bi) B.work.push_back(SWork{bi, e});
-        p0 = p1;
+    // most of their union tiles -- read the same slice of those tiles in consecutive items; the
+    // blocks of each team size together
+    for (int cls = 0; cls < 3; ++cls) {
+        auto in_class = [&](SBlock const& blk) { return cls == (blk.E > 64 ? 0 : blk.E > 32 ? 1 : 2); };
+        const size_t first = B.work.size();
+        for (int32_t p0 = 0; p0 < int32_t(nb);) {
+            int32_t p1 = p0 + 1;
+            if (panel > 0)
+                while (p1 < int32_t(nb) && p1 - p0 < panel && B.blocks[size_t(p1)].E == B.blocks[size_t(p0)].E &&
+                       B.blocks[size_t(p1)].rows == B.blocks[size_t(p0)].rows)
+                    ++p1;
+            if (in_class(B.blocks[size_t(p0)]))
+                for (int32_t e = 0; e < B.blocks[size_t(p0)].E; e += SBLOCK_ELEMS)
+                    for (int32_t bi = p0; bi < p1; ++bi) B.work.push_back(SWork{bi, e});
+            p0 = p1;
+        }
+        require(B.work.size() < size_t(INT32_MAX), "S blocks: more than 2^31 work items");
+        (cls == 0 ? B.n_work.team : cls == 1 ? B.n_work.pair : B.n_work.solo) = int32_t(B.work.size() - first);
+        // the items of one or two waves: longest k-step lists first (they run from a few to several
+        // hundred k-steps, each wave alone with its list)
+        if (cls > 0)
+            std::stable_sort(B.work.begin() + int64_t(first), B.work.end(), [&](SWork const& x, SWork const& y) {
+                return B.blocks[size_t(x.blk)].nk > B.blocks[size_t(y.blk)].nk;
+            });
+    }
+    // Launch list.  Workgroup i runs on XCD i mod 8: every 32 team items are dealt so that four
+    // consecutive ones (neighbouring element ranges, which share cache lines of T and S at their
+    // ends) run on one XCD.  The workgroups of smaller items wait on memory rather than use it, so
+    // they are spread, eight at a time, over the first eighth of the team items, whose work they
+    // overlap, and the long lists among them are done well before the end.
+    {
+        const int64_t nt = B.n_work.team, np = B.n_work.pair, ns = B.n_work.solo;
+        std::vector<SWork> small;
+        for (int64_t i = 0; i < ns; i += SB_WAVES) small.push_back(SWork{-1, int32_t(nt + np + i)});
+        for (int64_t i = 0; i < np; i += SB_WAVES / 2) small.push_back(SWork{-2, int32_t(nt + i)});
+        B.launch.reserve(size_t(nt) + small.size());
+        size_t q = 0;
+        for (int64_t i0 = 0; i0 < nt; i0 += 32) {
+            while (q < small.size() && int64_t(q) * (nt / 8) <= i0 * int64_t(small.size()))
+                for (int k = 0; k < 8 && q < small.size(); ++k) B.launch.push_back(small[q++]);
+            if (i0 + 32 <= nt)
+                for (int64_t r = 0; r < 32; ++r) B.launch.push_back(B.work[size_t(i0 + (r % 8) * 4 + r / 8)]);
+            else
+                B.launch.insert(B.launch.end(), B.work.begin() + i0, B.work.begin() + nt);
+        }
+        B.launch.insert(B.launch.end(), small.begin() + int64_t(q), small.end());
     }
     for (int32_t bi = 0; bi < int32_t(nb); ++bi) {
         SBlock const& blk = B.blocks[size_t(bi)];
@@ -1685,17 +1721,49 @@ void check_sblocks(SBlockTable const& B, uint64_t t_size, uint64_t s_size) {
         for (size_t bi = 0; bi < B.blocks.size(); ++bi)
             first[bi + 1] = first[bi] + uint64_t((B.blocks[bi].E + SBLOCK_ELEMS - 1) / SBLOCK_ELEMS);
         std::vector<char> seen(first.back(), 0);
-        if (B.work.size() != first.back()) bad = std::max(bad, 4);
-        for (SWork const& w : B.work) {
+        if (B.work.size() != first.back() || B.n_work.team < 0 || B.n_work.pair < 0 || B.n_work.solo < 0 ||
+            uint64_t(B.n_work.team) + uint64_t(B.n_work.pair) + uint64_t(B.n_work.solo) != B.work.size())
+            bad = std::max(bad, 4);
+        for (size_t i = 0; i < B.work.size(); ++i) {
+            SWork const& w = B.work[i];
             if (!(w.blk >= 0 && size_t(w.blk) < B.blocks.size() && w.n0 >= 0 && w.n0 < B.blocks[size_t(w.blk)].E &&
                   w.n0 % SBLOCK_ELEMS == 0)) {
                 bad = std::max(bad, 4);
                 continue;
             }
+            // an item of fewer waves than its tile needs would leave elements unwritten
+            const int32_t E = B.blocks[size_t(w.blk)].E;
+            if (i >= size_t(B.n_work.team) && (E > 64 || (i >= size_t(B.n_work.team) + size_t(B.n_work.pair) && E > 32)))
+                bad = std::max(bad, 4);
             char& c = seen[first[size_t(w.blk)] + uint64_t(w.n0 / SBLOCK_ELEMS)];
             if (c) bad = std::max(bad, 4);
             c = 1;
         }
+    }
+    // every work item in exactly one launch entry
+    if (bad == 0) {
+        const int64_t nt = B.n_work.team, np = B.n_work.pair, n = int64_t(B.work.size());
+        uint64_t teams = 0, items = 0;
+        std::vector<char> small(size_t(n - nt), 0);
+        for (SWork const& l : B.launch) {
+            if (l.blk >= 0) {
+                ++teams;
+                if (size_t(l.blk) >= B.blocks.size() || B.blocks[size_t(l.blk)].E <= 64 || l.n0 < 0 ||
+                    l.n0 >= B.blocks[size_t(l.blk)].E || l.n0 % SBLOCK_ELEMS != 0)
+                    bad = std::max(bad, 4);
+                continue;
+            }
+            const int64_t lo = l.blk == -1 ? nt + np : nt, hi = l.blk == -1 ? n : nt + np;
+            if (l.blk < -2 || l.n0 < lo || l.n0 >= hi) {
+                bad = std::max(bad, 4);
+                continue;
+            }
+            for (int64_t i = l.n0; i < std::min<int64_t>(hi, l.n0 + (l.blk == -1 ? SB_WAVES : SB_WAVES / 2)); ++i, ++items) {
+                if (small[size_t(i - nt)]) bad = std::max(bad, 4);
+                small[size_t(i - nt)] = 1;
+            }
+        }
+        if (teams != uint64_t(nt) || items != uint64_t(n - nt)) bad = std::max(bad, 4);
     }
     // small-tile tables: 5 malformed line, 6 term tile outside T, 7 malformed work item
     const int64_t nsl = int64_t(B.small_lines.size());

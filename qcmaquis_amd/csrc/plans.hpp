@@ -117,8 +117,16 @@ struct SBlock {
 };
 static_assert(sizeof(SBlock) == 40, "SBlock layout");
 struct SWork {
-    int32_t blk, n0;          // block and first tile element of one workgroup
+    int32_t blk, n0;          // block and first tile element of one work item
 };
+// Work items by the waves that share one: tiles of more than 64 elements on the four waves of a
+// workgroup, of 33 to 64 on two, of at most 32 on one; the work list holds them in this order.  The
+// launch list has one entry per workgroup: a team's work item itself, or for workgroups of smaller
+// items (blk < 0) the first of its items (work[n0]) with -blk = 1 (one wave each) or 2.
+struct SWorkCounts {
+    int32_t team = 0, pair = 0, solo = 0;
+};
+constexpr int SB_WAVES = 4;  // waves of a term-sum workgroup
 // Lines marked SLINE_SMALL (tiles of at most SMALL_LINE_LANES elements) are summed term by term:
 // each line gets a power-of-two group of lanes (one lane per tile element) and a workgroup of 256
 // lanes takes 256 / group consecutive lines of one group size (lines sorted by group size, then by
@@ -130,6 +138,8 @@ struct SSmallWork {
 struct SBlockTable {
     std::vector<SBlock> blocks;
     std::vector<SWork> work;
+    SWorkCounts n_work;           // the work items by team size
+    std::vector<SWork> launch;    // one entry per workgroup
     HostTable<int64_t> utile;     // T element offset of each union tile slot (-1: empty slot)
     HostTable<uint32_t> kstep;    // k-step words
     HostTable<double> ualpha;     // coefficient sub-blocks
@@ -159,7 +169,9 @@ std::vector<TermGradWork> term_grad_work(HostTable<SLine> const& lines, size_t l
 // lanes of a workgroup of the small-tile term sum; tiles up to this many elements can go there
 constexpr int SMALL_LINE_LANES = 256;
 // work items cover SBLOCK_ELEMS consecutive tile elements of one block
-constexpr int SBLOCK_ELEMS = 256;
+constexpr int SBLOCK_ELEMS = 128;
+// the block term sum loads one element past a tile of odd size: T buffers are that much longer
+constexpr int SB_T_SPARE = 2;
 
 // Execution schedule of a grouped GEMM stage.  Output tiles come in six shapes (BM x BN):
 // 32x128 for M <= 32, 64x64 for M <= 64, 96x64 for M <= 96 (problems without a row table), 128x64

@@ -1,0 +1,40 @@
+"""The block-form MPO-term sum at the edges of its work splits, against the CPU oracle: tiles of
+s x s elements with s*s around 32 (one wave), 64 (two waves) and 128 (a workgroup's range), single
+elements, odd sizes (an element pair past the tile's end) and coefficient tables longer than one
+staging pass.  FP64 to 1e-12 of the largest element (sums of a few thousand products, 2^-53 each),
+FP32 to 1e-5 (the mixed-precision bound of the other parity tests)."""
+import numpy as np
+import pytest
+
+from qcmaquis_amd import abi
+from qcmaquis_amd.engine import DeviceBoundary, DeviceMPO, HpsiPlan
+from qcmaquis_amd.synthetic import TWOU1_SITE, Chain, fuse_index
+from tests.chains import oracle_left, oracle_right, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("s,D", [(s, 24) for s in (1, 2, 5, 6, 8, 9, 11, 12, 17)] + [(1, 64), (12, 64)])
+def test_block_sum_tile_sizes(oracle_lib, ctx2u1, s, D):
+    ch = Chain(np.random.default_rng(100 + s), abi.MQ_SYM_TWOU1, 4, (4, 4), s, D,
+               phys=fuse_index(TWOU1_SITE, TWOU1_SITE), density=0.5, min_m=s)
+    k = 2
+    L = oracle_left(oracle_lib, ch, k)[k]
+    R = oracle_right(oracle_lib, ch, k + 1)[k + 1]
+    lay = ch.layouts[k]
+    psi = np.random.default_rng(s).normal(size=lay.n)
+    ref = oracle_lib.hpsi(ch.sym, ch.mpos[k], L, R, lay, psi)
+    ctx2u1.set_option(abi.MQ_OPT_SMALL_TILE_MAX, 0)  # every tile in blocks
+    try:
+        plan = HpsiPlan(ctx2u1, DeviceMPO(ctx2u1, ch.mpos[k]), DeviceBoundary.upload(ctx2u1, L),
+                        DeviceBoundary.upload(ctx2u1, R), lay)
+    finally:
+        ctx2u1.set_option(abi.MQ_OPT_SMALL_TILE_MAX, abi.MQ_SMALL_TILE_AUTO)
+    st = plan.stats()
+    err = rel_err(plan.apply(psi), ref)
+    err32 = rel_err(plan.apply(psi, abi.MQ_PREC_FP32), ref)
+    print(f"tiles {s}x{s}: {st['n_sblocks']} blocks, max union {st['max_union_tiles']}, FP64 {err:.1e}, FP32 {err32:.1e}",
+          flush=True)
+    assert st["small_lines"] == 0 and st["n_sblocks"] > 0
+    assert D < 64 or st["max_union_tiles"] > 4 * 64  # more k-steps than one staging pass holds
+    assert err < 1e-12 and err32 < 1e-5
