@@ -852,7 +852,7 @@ static void run_growth(mq_ctx_t ctx, GrowPlanHost& P, double const* bnd, double 
     GemmStage tg, cg;
     SAsmStage sa;
     try {
-        tg.upload(P.t_gemms, P.t_rows, ctx->stream);
+        tg.upload(fold_batches(P.t_gemms), P.t_rows, ctx->stream);
         cg.upload(P.c_gemms, {}, ctx->stream);
         sa.upload(SB, ctx->stream, ctx->sblock_xcd);
         st.seconds_upload = seconds_since(t);
@@ -1064,6 +1064,7 @@ static void finish_plan(mq_ctx_t ctx, mq_hpsi_plan_s* p, std::vector<LpanelPart>
         cgs[c].assign(H.c_gemms.begin() + int64_t(ch.c_gemm0), H.c_gemms.begin() + int64_t(ch.c_gemm1));
         check_gemms(tgs[c], sizes, trs[c]);
         check_gemms(cgs[c], sizes);
+        tgs[c] = fold_batches(tgs[c]);
         HostTable<SLine> cl(H.lines.begin() + int64_t(ch.line0), H.lines.begin() + int64_t(ch.line1));
         check_lines(cl, H.terms, ch.t_elems, ch.s_elems);
         auto tb = std::chrono::steady_clock::now();

@@ -1,8 +1,8 @@
 // gfx950 kernels of the contraction path.
 //
 //  * gemm_kernel: grouped, batched FP64 / FP32 GEMM over a host-built tile table.  32x128, 64x64,
-//    96x64 or 128x64 output tiles per 256-thread workgroup (four wave64s in a 2x2 grid, each a block of
-//    16x16x4 matrix-core tiles), operands staged through LDS in K-slices of 8 with the next slice
+//    96x64 or 128x64 output tiles per 256-thread workgroup (four wave64s in a 2x2 grid), wider ones
+//    in stages split along K; operands staged through LDS in K-slices of 8 with the next slice
 //    prefetched into registers.  Each output tile is owned by one workgroup or, when K is
 //    split, by a fixed set of partial tiles summed in order by gemm_reduce_kernel: no atomics.
 //  * sblock_kernel: the MPO-term sum (reference create_s / create_s_r, solver/tasks.cpp:425-494)
@@ -21,9 +21,6 @@ typedef double double4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
 namespace {
-
-constexpr int BK = 16;
-constexpr int LDS_PAD = 1;
 
 // The 16x16x4 matrix-core step of each compute precision.  Operands (measured on gfx950): lane l
 // supplies A[l % 16][l / 16] and B[l / 16][l % 16]; accumulator register r of lane l holds
@@ -61,81 +58,114 @@ __device__ inline void split_bf16(float x, short& hi, short& lo) {
 }
 
 // One BM x BN output tile (BM = 32 FM, BN = 16 FN WN) per workgroup of 2 WN waves; the waves form a
-// 2 x WN grid of 16 FM x 16 FN wave tiles, each FM x FN matrix-core tiles.  Operands of type TI,
-// computed in TI, output converted to TO.  The tile reduces over [k0, k1) and writes C, or its
-// partial tile (type TI) into the workspace (split K).
-template <int FM, int FN, class TI, class TO, int KS = BK, int MINB = 1, int WN = 2, bool BF3 = false>
-__global__ __launch_bounds__(128 * WN, MINB) void gemm_kernel(const GemmDesc* __restrict__ probs,
-                                                              const GemmRow* __restrict__ rows,
-                                                              const GemmTile* __restrict__ tiles, Bases bases,
-                                                              TI* __restrict__ ws) {
+// 2 x WN grid and take every second 16-row and every WN-th 16-column step of the tile, so a tile
+// cut short by the end of C leaves each of them its share.  Operands of type TI, computed in TI,
+// output converted to TO.  The tile reduces over [k0, k1) and writes C, or its partial tile (type
+// TI) into the workspace (split K).  K slices of KS go through two LDS buffers (one barrier per
+// slice), the next slice prefetched into registers.
+//
+// Every thread keeps pointers to the operand elements it stages and moves them on by a fixed step
+// per slice; rows and columns past the end of C read the last valid one (their products are not
+// stored), so only the last, shorter slice needs checks.  Matrix-core steps outside C, and k steps
+// of four outside the last slice, are skipped: sector sizes leave 0.2-0.8 of whole tiles useful, of
+// 16 x 16 x 4 steps 0.6-0.95.  T-GEMMs, FP64, checks per element and whole tiles -> now: 18 orbitals,
+// TwoU1, M = 509 0.51 -> 0.32 ms, M = 128 0.11 -> 0.04 ms; 20 orbitals, SU2U1, M = 2048 17.0 -> 14.8.
+template <int FM, int FN, class TI, int KS, int WN>
+struct GemmLds {
+    // rows padded so that the stores of a slice whose k runs across lanes meet every bank once
+    static constexpr int PAD = 16 / int(sizeof(TI));
+    TI A[2][KS][32 * FM + PAD];
+    TI B[2][KS][16 * FN * WN + PAD];
+};
+
+// the body of gemm_kernel for one orientation of its operands
+template <int FM, int FN, class TI, class TO, int KS, int WN, bool BF3, bool TA, bool TB>
+__device__ __forceinline__ void gemm_tile(GemmLds<FM, FN, TI, KS, WN>& lds, GemmTile const& tile, GemmDesc const& g,
+                                          const GemmRow* __restrict__ rows, Bases const& bases, TI* __restrict__ ws) {
     constexpr int THREADS = 128 * WN;
     constexpr int BM = 32 * FM, BN = 16 * FN * WN;
     constexpr int NA = BM * KS / THREADS, NB = BN * KS / THREADS;  // operand elements staged per thread and K slice
-    static_assert(KS % 4 == 0 && NA * THREADS == BM * KS && NB * THREADS == BN * KS, "K slice geometry");
+    static_assert(KS % 4 == 0 && NA * THREADS == BM * KS && NB * THREADS == BN * KS && THREADS % KS == 0 && THREADS % BN == 0,
+                  "K slice geometry");
     static_assert(!BF3 || (std::is_same<TI, float>::value && KS % 16 == 0), "split-BF16 products: FP32 operands, K slices of 16");
-    __shared__ TI As[KS][BM + LDS_PAD];
-    __shared__ TI Bs[KS][BN + LDS_PAD];
     typedef typename Mma<TI>::acc_t acc_t;
-
-    const GemmTile tile = tiles[blockIdx.x];
-    const GemmDesc g = probs[tile.prob];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    const int fr = lane & 15, fk = lane >> 4;
     const int m0 = tile.tm * BM, n0 = tile.tn * BN;
-    const bool ta = g.flags & GEMM_TRANS_A, tb = g.flags & GEMM_TRANS_B, rmap = g.flags & GEMM_ROWMAP;
-
+    const int ml = g.M - m0 < BM ? g.M - m0 : BM, nl = g.N - n0 < BN ? g.N - n0 : BN;  // rows and columns inside C
+    const bool rmap = !TA && (g.flags & GEMM_ROWMAP);
     const TI* A = static_cast<const TI*>(bases.p[g.base_a]) + (rmap ? 0 : g.a + int64_t(tile.batch) * g.sa);
     const TI* B = static_cast<const TI*>(bases.p[g.base_b]) + g.b + int64_t(tile.batch) * g.sb;
-    // stacked problem: the tile's rows are staged in LDS once (the A loads and the C stores look them
-    // up there); A is not transposed, so each thread loads from one row (tid % BM) of the tile
-    // (stacked problems only get tile heights that divide the workgroup size)
-    __shared__ GemmRow Rs[BM];
-    const TI* a_row = A;
-    int64_t a_rld = 0;
-    if (rmap) {
-        for (int i = tid; i < BM; i += THREADS)
-            if (m0 + i < g.M) Rs[i] = rows[g.a + m0 + i];
-        __syncthreads();
-        if (m0 + tid % BM < g.M) {
-            a_row = A + Rs[tid % BM].a;
-            a_rld = Rs[tid % BM].ld;
-        }
-    }
 
-    // per-thread load coordinates inside the BM x 16 A slice and the 16 x BN B slice, with the
-    // contiguous dimension of the operand across consecutive threads
-    int a_m[NA], a_k[NA], b_k[NB], b_n[NB];
+    // element i of this thread in the BM x KS slice of A: the contiguous dimension of the operand
+    // runs across consecutive threads.  Rows along threads (not transposed): with BM dividing the
+    // workgroup every element of a thread is of one row, k ADK apart, so one pointer walks through
+    // them.  k along threads: one k, a pointer per row.  The KS x BN slice of B likewise.
+    constexpr bool AWALK = !TA && THREADS % BM == 0;
+    constexpr int ADK = AWALK ? THREADS / BM : 0, ADM = THREADS / KS;
+    constexpr int BDK = THREADS / BN, BDN = THREADS / KS;
+    auto a_m = [&](int i) { return TA ? tid / KS + ADM * i : (tid + THREADS * i) % BM; };
+    auto a_k = [&](int i) { return TA ? tid % KS : (tid + THREADS * i) / BM; };
+    auto b_n = [&](int i) { return TB ? tid % BN : tid / KS + BDN * i; };
+    auto b_k = [&](int i) { return TB ? tid / BN + BDK * i : tid % KS; };
+    const TI *pa[AWALK ? 1 : NA], *pb[TB ? 1 : NB];
+    int64_t a_step, b_step;  // per element of a walk, else per slice
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
-        const int idx = tid + THREADS * i;
-        if (!ta) { a_m[i] = idx % BM; a_k[i] = idx / BM; }
-        else     { a_k[i] = idx % KS; a_m[i] = idx / KS; }
-    }
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-        const int idx = tid + THREADS * i;
-        if (!tb) { b_k[i] = idx % KS; b_n[i] = idx / KS; }
-        else     { b_n[i] = idx % BN; b_k[i] = idx / BN; }
-    }
-    const int k_end = tile.k1;
-    TI ra[NA], rb[NB];
-    auto load = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < NA; ++i) {
-            int m = m0 + a_m[i], k = k0 + a_k[i];
-            bool ok = (m < g.M) && (k < k_end);
-            const TI* pa = rmap ? a_row + int64_t(k) * a_rld
-                                : ta ? A + int64_t(m) * g.lda + k : A + m + int64_t(k) * g.lda;
-            ra[i] = ld_or_zero(pa, ok);
+    for (int i = 0; i < (AWALK ? 1 : NA); ++i) {
+        const int m = m0 + (a_m(i) < ml ? a_m(i) : ml - 1);
+        const int64_t k = tile.k0 + a_k(i);
+        if (rmap) {
+            const GemmRow r = rows[g.a + m];
+            pa[i] = A + r.a + k * r.ld;
+            a_step = int64_t(AWALK ? ADK : KS) * r.ld;
+        } else {
+            pa[i] = TA ? A + int64_t(m) * g.lda + k : A + m + k * g.lda;
+            a_step = TA ? KS : int64_t(AWALK ? ADK : KS) * g.lda;
         }
+    }
 #pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            int n = n0 + b_n[i], kb = k0 + b_k[i];
-            bool okb = (n < g.N) && (kb < k_end);
-            const TI* pb = tb ? B + n + int64_t(kb) * g.ldb : B + kb + int64_t(n) * g.ldb;
-            rb[i] = ld_or_zero(pb, okb);
+    for (int i = 0; i < (TB ? 1 : NB); ++i) {
+        const int n = n0 + (b_n(i) < nl ? b_n(i) : nl - 1);
+        const int64_t k = tile.k0 + b_k(i);
+        if (TB) {
+            // columns in blocks of g.nb, a block every g.sb elements
+            pb[i] = (g.flags & GEMM_NBLOCKS ? B + int64_t(n / g.nb) * g.sb + n % g.nb : B + n) + k * g.ldb;
+        } else {
+            pb[i] = B + k + int64_t(n) * g.ldb;
+        }
+    }
+    b_step = TB ? int64_t(BDK) * g.ldb : KS;
+    TI ra[NA], rb[NB];
+    auto load = [&](int kn) {  // the next kn <= KS values of k
+        if (kn >= KS) {
+#pragma unroll
+            for (int i = 0; i < NA; ++i) {
+                const TI*& p = pa[AWALK ? 0 : i];
+                ra[i] = *p;
+                p += a_step;
+            }
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const TI*& p = pb[TB ? 0 : i];
+                rb[i] = *p;
+                p += b_step;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < NA; ++i) {
+                const TI*& p = pa[AWALK ? 0 : i];
+                ra[i] = ld_or_zero(p, a_k(i) < kn);
+                p += a_step;
+            }
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const TI*& p = pb[TB ? 0 : i];
+                rb[i] = ld_or_zero(p, b_k(i) < kn);
+                p += b_step;
+            }
         }
     };
 
@@ -144,19 +174,11 @@ __global__ __launch_bounds__(128 * WN, MINB) void gemm_kernel(const GemmDesc* __
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
-
-    const int wm = (wave & 1) * 16 * FM, wn = (wave >> 1) * 16 * FN;
-    const int fr = lane & 15, fk = lane >> 4;
-
-    if (tile.k0 < k_end) load(tile.k0);
-    for (int k0 = tile.k0; k0 < k_end; k0 += KS) {
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < NA; ++i) As[a_k[i]][a_m[i]] = ra[i];
-#pragma unroll
-        for (int i = 0; i < NB; ++i) Bs[b_k[i]][b_n[i]] = rb[i];
-        __syncthreads();
-        if (k0 + KS < k_end) load(k0 + KS);
+    // matrix-core steps of this wave inside C
+    const int fm = (ml - 16 * wm + 31) / 32, fn = (nl - 16 * wn + 16 * WN - 1) / (16 * WN);
+    // operands swapped in every step: the instruction accumulates the transposed tile C^T = B^T A^T
+    auto multiply = [&](int buf, int kn, auto all) {
+        constexpr bool ALL = decltype(all)::value;
         if constexpr (BF3) {
 #pragma unroll
             for (int kk = 0; kk < KS; kk += 16) {
@@ -166,7 +188,7 @@ __global__ __launch_bounds__(128 * WN, MINB) void gemm_kernel(const GemmDesc* __
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
                         short h, l;
-                        split_bf16(As[kk + 4 * fk + q][wm + 16 * i + fr], h, l);
+                        split_bf16(lds.A[buf][kk + 4 * fk + q][16 * (2 * i + wm) + fr], h, l);
                         ah[i][q] = h;
                         al[i][q] = l;
                     }
@@ -175,36 +197,53 @@ __global__ __launch_bounds__(128 * WN, MINB) void gemm_kernel(const GemmDesc* __
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
                         short h, l;
-                        split_bf16(Bs[kk + 4 * fk + q][wn + 16 * j + fr], h, l);
+                        split_bf16(lds.B[buf][kk + 4 * fk + q][16 * (WN * j + wn) + fr], h, l);
                         bh[j][q] = h;
                         bl[j][q] = l;
                     }
-                // operands swapped as below: the instruction accumulates C^T = B^T A^T
 #pragma unroll
                 for (int i = 0; i < FM; ++i)
 #pragma unroll
-                    for (int j = 0; j < FN; ++j) {
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bh[j], ah[i], acc[i][j], 0, 0, 0);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bh[j], al[i], acc[i][j], 0, 0, 0);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bl[j], ah[i], acc[i][j], 0, 0, 0);
-                    }
+                    for (int j = 0; j < FN; ++j)
+                        if (ALL || (i < fm && j < fn)) {
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bh[j], ah[i], acc[i][j], 0, 0, 0);
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bh[j], al[i], acc[i][j], 0, 0, 0);
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bl[j], ah[i], acc[i][j], 0, 0, 0);
+                        }
             }
-            continue;
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < KS; kk += 4) {
+                if (kk < kn) {
+                    TI af[FM], bf[FN];
+#pragma unroll
+                    for (int i = 0; i < FM; ++i) af[i] = lds.A[buf][kk + fk][16 * (2 * i + wm) + fr];
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) bf[j] = lds.B[buf][kk + fk][16 * (WN * j + wn) + fr];
+#pragma unroll
+                    for (int i = 0; i < FM; ++i)
+#pragma unroll
+                        for (int j = 0; j < FN; ++j)
+                            if (ALL || (i < fm && j < fn)) acc[i][j] = Mma<TI>::step(bf[j], af[i], acc[i][j]);
+                }
+            }
         }
+    };
+    auto reduce = [&](auto all) {
+        int left = tile.k1 - tile.k0;
+        if (left > 0) load(left);
+        for (int buf = 0; left > 0; buf ^= 1, left -= KS) {
 #pragma unroll
-        for (int kk = 0; kk < KS; kk += 4) {
-            TI af[FM], bf[FN];
+            for (int i = 0; i < NA; ++i) lds.A[buf][a_k(i)][a_m(i)] = ra[i];
 #pragma unroll
-            for (int i = 0; i < FM; ++i) af[i] = As[kk + fk][wm + 16 * i + fr];
-#pragma unroll
-            for (int j = 0; j < FN; ++j) bf[j] = Bs[kk + fk][wn + 16 * j + fr];
-            // operands swapped: the instruction accumulates the transposed tile C^T = B^T A^T
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j) acc[i][j] = Mma<TI>::step(bf[j], af[i], acc[i][j]);
+            for (int i = 0; i < NB; ++i) lds.B[buf][b_k(i)][b_n(i)] = rb[i];
+            __syncthreads();
+            if (left > KS) load(left - KS);
+            multiply(buf, left, all);
         }
-    }
+    };
+    if (ml == BM && nl == BN) reduce(std::true_type());
+    else reduce(std::false_type());
 
     // D = C^T: register r of lane l holds C[l % 16][row(l, r)] of its 16 x 16 tile, so
     // consecutive lanes store consecutive rows of a column
@@ -212,13 +251,13 @@ __global__ __launch_bounds__(128 * WN, MINB) void gemm_kernel(const GemmDesc* __
     const bool split = tile.ws >= 0;  // never for stacked problems
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-        const int mm = wm + 16 * i + fr, m = m0 + mm;
-        if (m >= g.M) continue;
+        const int mm = 16 * (2 * i + wm) + fr, m = m0 + mm;
+        if (mm >= ml) continue;
         // column n of this row at c_row + n * c_ld
         TO* c_row = C + m;
         int64_t c_ld = g.ldc;
         if (rmap) {
-            const GemmRow r = Rs[mm];
+            const GemmRow r = rows[g.a + m];
             c_row = C + r.c + int64_t(tile.batch) * g.sc * r.ld;
             c_ld = r.ld;
         }
@@ -226,12 +265,30 @@ __global__ __launch_bounds__(128 * WN, MINB) void gemm_kernel(const GemmDesc* __
         for (int j = 0; j < FN; ++j) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                int nn = wn + 16 * j + Mma<TI>::row(lane, r), n = n0 + nn;
-                if (n >= g.N) continue;
+                const int nn = 16 * (WN * j + wn) + Mma<TI>::row(lane, r);
+                if (nn >= nl) continue;
                 if (split) ws[tile.ws + mm + int64_t(nn) * BM] = acc[i][j][r];
-                else c_row[int64_t(n) * c_ld] = TO(acc[i][j][r]);
+                else c_row[int64_t(n0 + nn) * c_ld] = TO(acc[i][j][r]);
             }
         }
+    }
+}
+
+template <int FM, int FN, class TI, class TO, int KS, int MINB = 1, int WN = 2, bool BF3 = false>
+__global__ __launch_bounds__(128 * WN, MINB) void gemm_kernel(const GemmDesc* __restrict__ probs,
+                                                              const GemmRow* __restrict__ rows,
+                                                              const GemmTile* __restrict__ tiles, Bases bases,
+                                                              TI* __restrict__ ws) {
+    __shared__ GemmLds<FM, FN, TI, KS, WN> lds;
+    const GemmTile tile = tiles[blockIdx.x];
+    const GemmDesc g = probs[tile.prob];
+    const bool tb = g.flags & GEMM_TRANS_B;
+    if (g.flags & GEMM_TRANS_A) {
+        if (tb) gemm_tile<FM, FN, TI, TO, KS, WN, BF3, true, true>(lds, tile, g, rows, bases, ws);
+        else gemm_tile<FM, FN, TI, TO, KS, WN, BF3, true, false>(lds, tile, g, rows, bases, ws);
+    } else {
+        if (tb) gemm_tile<FM, FN, TI, TO, KS, WN, BF3, false, true>(lds, tile, g, rows, bases, ws);
+        else gemm_tile<FM, FN, TI, TO, KS, WN, BF3, false, false>(lds, tile, g, rows, bases, ws);
     }
 }
 

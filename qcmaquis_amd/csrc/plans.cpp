@@ -1800,6 +1800,21 @@ void check_sblocks(SBlockTable const& B, uint64_t t_size, uint64_t s_size) {
     require(bad != 7, "S blocks: malformed small-tile work item");
 }
 
+std::vector<GemmDesc> fold_batches(std::vector<GemmDesc> const& v) {
+    std::vector<GemmDesc> out(v);
+    for (auto& g : out) {
+        // C row m, column n of block b at c + (n + b sc) ld: one run of columns when sc is N
+        if (g.batch <= 1 || !(g.flags & GEMM_ROWMAP) || !(g.flags & GEMM_TRANS_B) || g.sc != g.N || g.N <= 0 ||
+            int64_t(g.N) * g.batch >= INT32_MAX)
+            continue;
+        g.nb = g.N;
+        g.N *= g.batch;
+        g.batch = 1;
+        g.flags |= GEMM_NBLOCKS;
+    }
+    return out;
+}
+
 // ---- grouped GEMM schedule ---------------------------------------------------------------------
 GemmPolicy gemm_policy(int i) {
     require(i >= 0 && i < GEMM_N_POLICIES, "gemm policy: index out of range");

@@ -51,6 +51,7 @@ enum : int32_t {
     GEMM_TRANS_A = 1,
     GEMM_TRANS_B = 2,
     GEMM_ROWMAP = 4,  // stacked problem: rows from a row table (A not transposed, never split along K)
+    GEMM_NBLOCKS = 8, // columns in blocks of nb (B transposed): column n of B at (n / nb) sb + n % nb
 };
 enum : int32_t {  // operand base selectors
     BASE_PSI_IN = 0, BASE_PSI_OUT, BASE_T, BASE_S, BASE_LPANEL, BASE_BOUNDARY, BASE_BRA, BASE_KET,
@@ -63,9 +64,16 @@ struct GemmDesc {
     int32_t lda, ldb, ldc;
     int32_t flags;          // GEMM_TRANS_*
     int32_t base_a, base_b, base_c;
-    int32_t pad;
+    int32_t nb;             // GEMM_NBLOCKS: columns of a block
 };
 static_assert(sizeof(GemmDesc) == 96, "GemmDesc layout");
+
+// The stacked problems of a stage with their batch folded into the columns, for the device: T tasks
+// that read a right boundary transposed are one product per block of the cohort (nb of them, N
+// columns each, N often far below a tile's width), whose C columns follow each other; folded, a
+// tile takes columns of as many blocks as it holds (GEMM_NBLOCKS).  Other problems are returned as
+// they are.
+std::vector<GemmDesc> fold_batches(std::vector<GemmDesc> const& v);
 
 // Row of a stacked problem (GEMM_ROWMAP).  Several products that share their B operand (T-GEMMs
 // reading one right-boundary cohort) run as one problem whose M rows are the rows of their A

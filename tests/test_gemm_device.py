@@ -1,0 +1,50 @@
+"""The device form of the grouped GEMM stages against the plan's own problems, on the CPU."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+from qcmaquis_amd import abi
+from qcmaquis_amd.synthetic import TWOU1_SITE, fuse_index
+from tests import emu
+from tests.chains import make_chain, oracle_left, oracle_right
+
+LIB = os.path.join(emu.HERE, "libgemmdevice.so")
+
+
+@pytest.fixture(scope="module")
+def lib():
+    srcs = [os.path.join(emu.HERE, "gemm_device.cpp")] + [os.path.join(emu.CSRC, f) for f in
+                                                          ("plans.cpp", "coupling.cpp", "descriptors.cpp")]
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fopenmp", "-I", os.path.join(emu.ROOT, "include"),
+                    "-I", emu.CSRC, "-o", LIB] + srcs, check=True)
+    lib = C.CDLL(LIB)
+    idx = C.POINTER(abi.IndexDesc)
+    lib.fold_check.restype = C.c_long
+    lib.fold_check.argtypes = [C.c_int, C.POINTER(abi.MPODesc), C.POINTER(abi.BIndexDesc), C.POINTER(abi.BIndexDesc), idx,
+                               idx, idx]
+    return lib
+
+
+CHAINS = [
+    (abi.MQ_SYM_TWOU1, 1, dict(n_sites=5, total=(3, 2), max_m=1, D=6)),
+    (abi.MQ_SYM_TWOU1, 2, dict(n_sites=5, total=(3, 2), max_m=9, D=9)),
+    (abi.MQ_SYM_TWOU1, 3, dict(n_sites=4, total=(4, 4), max_m=7, D=12, phys=fuse_index(TWOU1_SITE, TWOU1_SITE))),
+    (abi.MQ_SYM_SU2U1, 4, dict(n_sites=5, total=(4, 0), max_m=6, D=9)),
+]
+
+
+def test_folded_batches(oracle_lib, lib):
+    folded = 0
+    for sym, seed, kw in CHAINS:
+        ch = make_chain(seed, sym=sym, **kw)
+        n = len(ch.mpos)
+        L, R = oracle_left(oracle_lib, ch, n - 1), oracle_right(oracle_lib, ch, 1)
+        for k in range(n):
+            lay = ch.layouts[k]
+            d = [ch.mpos[k].desc(), L[k].desc(), R[k + 1].desc(), lay.left.desc(), lay.phys.desc(), lay.right.desc()]
+            f = lib.fold_check(sym, *[C.byref(x) for x in d])
+            assert f >= 0, (sym, seed, k)
+            folded += f
+    assert folded > 0
