@@ -291,15 +291,17 @@ int guarded(mq_ctx_t ctx, F&& f) {
     }
 }
 
-// device copy of a grouped GEMM stage and its schedule (tiles per shape, split-K reduce jobs and
+// device copy of a grouped GEMM stage and its schedule (work items, split-K reduce jobs and
 // the workspace of the partial tiles, sized for FP64 and shared by the FP32 launches)
 struct GemmStage {
     GemmDesc* probs = nullptr;
     GemmRow* rows = nullptr;
-    GemmTile* tiles[GEMM_N_SHAPES] = {};
-    int64_t n_tiles[GEMM_N_SHAPES] = {};
+    GemmItem* items = nullptr;
+    int64_t n_items = 0;
     GemmReduce* reduces = nullptr;
     int64_t n_reduces = 0;
+    int32_t reduce_elems = 0;
+    bool trans_a = false;  // some problem reads A transposed (FP64 only)
     double* ws = nullptr;
     bool own_ws = true;
     // sch: the stage's schedule (built here when null); ws_shared: a split-K workspace of at least
@@ -314,23 +316,31 @@ struct GemmStage {
         GemmSchedule const& sch = *pre;
         probs = dev_upload(v, s);
         rows = dev_upload(r, s);
-        for (int sh = 0; sh < GEMM_N_SHAPES; ++sh) {
-            tiles[sh] = dev_upload(sch.tiles[sh], s);
-            n_tiles[sh] = int64_t(sch.tiles[sh].size());
+        trans_a = false;
+        for (GemmDesc const& g : v) {
+            require((g.flags & (GEMM_TRANS_A | GEMM_TRANS_B)) != (GEMM_TRANS_A | GEMM_TRANS_B), "gemm stage: both operands transposed");
+            trans_a |= (g.flags & GEMM_TRANS_A) != 0;
         }
+        const std::vector<GemmItem> list = gemm_items(v, sch);
+        items = dev_upload(list, s);
+        n_items = int64_t(list.size());
         reduces = dev_upload(sch.reduces, s);
         n_reduces = int64_t(sch.reduces.size());
+        reduce_elems = 0;
+        for (GemmReduce const& j : sch.reduces) reduce_elems = std::max(reduce_elems, gemm_bm(j.shape) * gemm_bn(j.shape));
         own_ws = ws_shared == nullptr;
         ws = own_ws ? dev_alloc<double>(sch.ws_elems) : ws_shared;
     }
     void run(Bases const& b, hipStream_t s, GemmPrec prec) const {
-        hipcheck(launch_gemm(prec, probs, rows, tiles, n_tiles, reduces, n_reduces, ws, b, s), "gemm launch");
+        require(!trans_a || prec == GEMM_F64, "gemm stage: transposed A operands are FP64");
+        hipcheck(launch_gemm(prec, probs, rows, items, n_items, reduces, n_reduces, reduce_elems, ws, b, s), "gemm launch");
     }
     void release() {
         dev_free(probs);
         dev_free(rows);
         rows = nullptr;
-        for (auto& t : tiles) dev_free(t), t = nullptr;
+        dev_free(items);
+        items = nullptr;
         dev_free(reduces);
         if (own_ws) dev_free(ws);
         probs = nullptr;

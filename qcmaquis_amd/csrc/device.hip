@@ -1,10 +1,10 @@
 // gfx950 kernels of the contraction path.
 //
-//  * gemm_kernel: grouped, batched FP64 / FP32 GEMM over a host-built tile table.  32x128, 64x64,
-//    96x64 or 128x64 output tiles per 256-thread workgroup (four wave64s in a 2x2 grid), wider ones
-//    in stages split along K; operands staged through LDS in K-slices of 8 with the next slice
-//    prefetched into registers.  Each output tile is owned by one workgroup or, when K is
-//    split, by a fixed set of partial tiles summed in order by gemm_reduce_kernel: no atomics.
+//  * gemm_kernel: grouped, batched FP64 / FP32 GEMM over a host-built list of work items of up to
+//    128 rows and 128 columns, stages with few of them split along K; eight wave64s of 16 columns
+//    each, operands staged through LDS in K slices of 16 with the next slice prefetched into
+//    registers.  Each output tile is owned by one workgroup or, when K is split, by a fixed set of
+//    partial tiles summed in order by gemm_reduce_kernel: no atomics.
 //  * sblock_kernel: the MPO-term sum (reference create_s / create_s_r, solver/tasks.cpp:425-494)
 //    as a block-sparse product on the matrix cores: up to 64 output tiles ("lines") of equal shape
 //    at a time, in groups of 16, Y_g = alpha_g * X over the union of the T tiles they read, each
@@ -57,246 +57,219 @@ __device__ inline void split_bf16(float x, short& hi, short& lo) {
     lo = short((r + 0x7fffu + ((r >> 16) & 1u)) >> 16);
 }
 
-// One BM x BN output tile (BM = 32 FM, BN = 16 FN WN) per workgroup of 2 WN waves; the waves form a
-// 2 x WN grid and take every second 16-row and every WN-th 16-column step of the tile, so a tile
-// cut short by the end of C leaves each of them its share.  Operands of type TI, computed in TI,
-// output converted to TO.  The tile reduces over [k0, k1) and writes C, or its partial tile (type
-// TI) into the workspace (split K).  K slices of KS go through two LDS buffers (one barrier per
-// slice), the next slice prefetched into registers.
+// Grouped GEMM.  A workgroup of eight waves computes one work item: up to 128 rows and 128 columns of a
+// problem's C, operands of type TI, computed in TI, output converted to TO, reduced over [k0, k1) and
+// written to C or, as a partial tile (type TI), into the workspace (split K).  A wave owns 16 columns
+// and all rows of the item, in 16-row steps, so the waves share the work evenly however many rows
+// there are; steps of rows outside the item, and k steps of four outside the last slice, are
+// skipped.  K slices of 16 go through two LDS buffers (one barrier per slice), the next slice
+// prefetched into registers.
 //
 // Every thread keeps pointers to the operand elements it stages and moves them on by a fixed step
 // per slice; rows and columns past the end of C read the last valid one (their products are not
-// stored), so only the last, shorter slice needs checks.  Matrix-core steps outside C, and k steps
-// of four outside the last slice, are skipped: sector sizes leave 0.2-0.8 of whole tiles useful, of
-// 16 x 16 x 4 steps 0.6-0.95.  T-GEMMs, FP64, checks per element and whole tiles -> now: 18 orbitals,
-// TwoU1, M = 509 0.51 -> 0.32 ms, M = 128 0.11 -> 0.04 ms; 20 orbitals, SU2U1, M = 2048 17.0 -> 14.8.
-template <int FM, int FN, class TI, int KS, int WN>
+// stored), so only the last, shorter slice needs checks.
+//
+// Bound: the FP64 matrix cores in stages of large sectors (L*S of 20 orbitals and M = 2048: 48 TFLOP/s of
+// useful work, of 71 in a dense product of 8192), the stores of T rows and the latency of an item's
+// few K slices elsewhere.  Against 256 threads on 32x128, 64x64, 96x64 and 128x64 tiles, one launch
+// per tile shape: B is staged for 128 columns of up to 128 rows instead of 64, waves of an item
+// no longer wait for the one with the most row steps, and the items of all heights share one launch
+// and one tail.  T / L*S stages in us before -> now: 8 orbitals, M = 40 8 / 23 -> 8 / 20;
+// 18, M = 509 323 / 412 -> 307 / 400; 20 with spins, M = 700 997 / 958 -> 913 / 901, M = 2048
+// 14.8 / 18.9 -> 13.8 / 15.1 ms.
+constexpr int GEMM_TILE = 128, GEMM_KS = 16, GEMM_THREADS = 512;
+template <class TI>
 struct GemmLds {
     // rows padded so that the stores of a slice whose k runs across lanes meet every bank once
-    static constexpr int PAD = 16 / int(sizeof(TI));
-    TI A[2][KS][32 * FM + PAD];
-    TI B[2][KS][16 * FN * WN + PAD];
+    static constexpr int PAD = 8 / int(sizeof(TI));
+    TI A[2][GEMM_KS][GEMM_TILE + PAD];
+    TI B[2][GEMM_KS][GEMM_TILE + PAD];
+    int64_t row_c[GEMM_TILE];  // stacked problems: C offset and leading dimension of every row
+    int32_t row_ld[GEMM_TILE];
 };
 
 // the body of gemm_kernel for one orientation of its operands
-template <int FM, int FN, class TI, class TO, int KS, int WN, bool BF3, bool TA, bool TB>
-__device__ __forceinline__ void gemm_tile(GemmLds<FM, FN, TI, KS, WN>& lds, GemmTile const& tile, GemmDesc const& g,
+template <class TI, class TO, bool BF3, bool TA, bool TB>
+__device__ __forceinline__ void gemm_tile(GemmLds<TI>& lds, GemmItem const& tile, GemmDesc const& g,
                                           const GemmRow* __restrict__ rows, Bases const& bases, TI* __restrict__ ws) {
-    constexpr int THREADS = 128 * WN;
-    constexpr int BM = 32 * FM, BN = 16 * FN * WN;
-    constexpr int NA = BM * KS / THREADS, NB = BN * KS / THREADS;  // operand elements staged per thread and K slice
-    static_assert(KS % 4 == 0 && NA * THREADS == BM * KS && NB * THREADS == BN * KS && THREADS % KS == 0 && THREADS % BN == 0,
-                  "K slice geometry");
-    static_assert(!BF3 || (std::is_same<TI, float>::value && KS % 16 == 0), "split-BF16 products: FP32 operands, K slices of 16");
+    constexpr int KS = GEMM_KS, THREADS = GEMM_THREADS, BT = GEMM_TILE, F = BT / 16;
+    constexpr int NE = BT * KS / THREADS;  // elements of each operand staged per thread and K slice
+    static_assert(NE * THREADS == BT * KS && THREADS % BT == 0 && THREADS % KS == 0 && THREADS == 64 * F, "K slice geometry");
+    static_assert(!BF3 || std::is_same<TI, float>::value, "split-BF16 products: FP32 operands");
     typedef typename Mma<TI>::acc_t acc_t;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave & 1, wn = wave >> 1;
     const int fr = lane & 15, fk = lane >> 4;
-    const int m0 = tile.tm * BM, n0 = tile.tn * BN;
-    const int ml = g.M - m0 < BM ? g.M - m0 : BM, nl = g.N - n0 < BN ? g.N - n0 : BN;  // rows and columns inside C
+    const int m0 = tile.m0, n0 = tile.n0;
+    const int ml = tile.ml, nl = g.N - n0 < BT ? g.N - n0 : BT;  // rows and columns of the item
     const bool rmap = !TA && (g.flags & GEMM_ROWMAP);
     const TI* A = static_cast<const TI*>(bases.p[g.base_a]) + (rmap ? 0 : g.a + int64_t(tile.batch) * g.sa);
     const TI* B = static_cast<const TI*>(bases.p[g.base_b]) + g.b + int64_t(tile.batch) * g.sb;
 
-    // element i of this thread in the BM x KS slice of A: the contiguous dimension of the operand
-    // runs across consecutive threads.  Rows along threads (not transposed): with BM dividing the
-    // workgroup every element of a thread is of one row, k ADK apart, so one pointer walks through
-    // them.  k along threads: one k, a pointer per row.  The KS x BN slice of B likewise.
-    constexpr bool AWALK = !TA && THREADS % BM == 0;
-    constexpr int ADK = AWALK ? THREADS / BM : 0, ADM = THREADS / KS;
-    constexpr int BDK = THREADS / BN, BDN = THREADS / KS;
-    auto a_m = [&](int i) { return TA ? tid / KS + ADM * i : (tid + THREADS * i) % BM; };
-    auto a_k = [&](int i) { return TA ? tid % KS : (tid + THREADS * i) / BM; };
-    auto b_n = [&](int i) { return TB ? tid % BN : tid / KS + BDN * i; };
-    auto b_k = [&](int i) { return TB ? tid / BN + BDK * i : tid % KS; };
-    const TI *pa[AWALK ? 1 : NA], *pb[TB ? 1 : NB];
-    int64_t a_step, b_step;  // per element of a walk, else per slice
+    // element i of this thread in a slice: the contiguous dimension of the operand runs across
+    // consecutive threads.  Rows (columns) along threads: all of one row, DK apart in k, so one
+    // pointer walks through them.  k along threads: all of one k, a pointer per row, DM apart.
+    constexpr int DK = THREADS / BT, DM = THREADS / KS;
+    auto a_m = [&](int i) { return TA ? tid / KS + DM * i : tid % BT; };
+    auto a_k = [&](int i) { return TA ? tid % KS : tid / BT + DK * i; };
+    auto b_n = [&](int i) { return TB ? tid % BT : tid / KS + DM * i; };
+    auto b_k = [&](int i) { return TB ? tid / BT + DK * i : tid % KS; };
+    const TI *pa[TA ? NE : 1], *pb[TB ? 1 : NE];
+    int64_t a_step = 0, b_step;  // per element of a walk, else per slice
 #pragma unroll
-    for (int i = 0; i < (AWALK ? 1 : NA); ++i) {
+    for (int i = 0; i < (TA ? NE : 1); ++i) {
         const int m = m0 + (a_m(i) < ml ? a_m(i) : ml - 1);
         const int64_t k = tile.k0 + a_k(i);
         if (rmap) {
             const GemmRow r = rows[g.a + m];
             pa[i] = A + r.a + k * r.ld;
-            a_step = int64_t(AWALK ? ADK : KS) * r.ld;
+            a_step = int64_t(DK) * r.ld;
+            if (tid < BT) {
+                lds.row_c[tid] = r.c;
+                lds.row_ld[tid] = r.ld;
+            }
         } else {
             pa[i] = TA ? A + int64_t(m) * g.lda + k : A + m + k * g.lda;
-            a_step = TA ? KS : int64_t(AWALK ? ADK : KS) * g.lda;
+            a_step = TA ? KS : int64_t(DK) * g.lda;
         }
     }
 #pragma unroll
-    for (int i = 0; i < (TB ? 1 : NB); ++i) {
+    for (int i = 0; i < (TB ? 1 : NE); ++i) {
         const int n = n0 + (b_n(i) < nl ? b_n(i) : nl - 1);
         const int64_t k = tile.k0 + b_k(i);
-        if (TB) {
-            // columns in blocks of g.nb, a block every g.sb elements
+        if (TB)  // columns in blocks of g.nb, a block every g.sb elements
             pb[i] = (g.flags & GEMM_NBLOCKS ? B + int64_t(n / g.nb) * g.sb + n % g.nb : B + n) + k * g.ldb;
-        } else {
+        else
             pb[i] = B + k + int64_t(n) * g.ldb;
-        }
     }
-    b_step = TB ? int64_t(BDK) * g.ldb : KS;
-    TI ra[NA], rb[NB];
+    b_step = TB ? int64_t(DK) * g.ldb : KS;
+    TI ra[NE], rb[NE];
     auto load = [&](int kn) {  // the next kn <= KS values of k
-        if (kn >= KS) {
+        const bool whole = kn >= KS;
 #pragma unroll
-            for (int i = 0; i < NA; ++i) {
-                const TI*& p = pa[AWALK ? 0 : i];
-                ra[i] = *p;
-                p += a_step;
-            }
+        for (int i = 0; i < NE; ++i) {
+            const TI*& p = pa[TA ? i : 0];
+            ra[i] = whole ? *p : ld_or_zero(p, a_k(i) < kn);
+            p += a_step;
+        }
 #pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                const TI*& p = pb[TB ? 0 : i];
-                rb[i] = *p;
-                p += b_step;
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < NA; ++i) {
-                const TI*& p = pa[AWALK ? 0 : i];
-                ra[i] = ld_or_zero(p, a_k(i) < kn);
-                p += a_step;
-            }
-#pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                const TI*& p = pb[TB ? 0 : i];
-                rb[i] = ld_or_zero(p, b_k(i) < kn);
-                p += b_step;
-            }
+        for (int i = 0; i < NE; ++i) {
+            const TI*& p = pb[TB ? 0 : i];
+            rb[i] = whole ? *p : ld_or_zero(p, b_k(i) < kn);
+            p += b_step;
         }
     };
 
-    acc_t acc[FM][FN];
+    acc_t acc[F];
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
-    // matrix-core steps of this wave inside C
-    const int fm = (ml - 16 * wm + 31) / 32, fn = (nl - 16 * wn + 16 * WN - 1) / (16 * WN);
-    // operands swapped in every step: the instruction accumulates the transposed tile C^T = B^T A^T
-    auto multiply = [&](int buf, int kn, auto all) {
+    for (int i = 0; i < F; ++i) acc[i] = acc_t{0, 0, 0, 0};
+    const int fm = (ml + 15) / 16;  // row steps of the item
+    const int wc = 16 * wave;       // first column of this wave
+    // one slice: S row steps, of which the first fm count unless ALL do.  Operands swapped in every
+    // step: the instruction accumulates the transposed tile C^T = B^T A^T
+    auto multiply = [&](int buf, int kn, auto steps, auto all) {
+        constexpr int S = decltype(steps)::value;
         constexpr bool ALL = decltype(all)::value;
         if constexpr (BF3) {
+            bf16x4_t bh, bl;
 #pragma unroll
-            for (int kk = 0; kk < KS; kk += 16) {
-                bf16x4_t ah[FM], al[FM], bh[FN], bl[FN];
+            for (int q = 0; q < 4; ++q) {
+                short h, l;
+                split_bf16(lds.B[buf][4 * fk + q][wc + fr], h, l);
+                bh[q] = h;
+                bl[q] = l;
+            }
 #pragma unroll
-                for (int i = 0; i < FM; ++i)
+            for (int i = 0; i < S; ++i) {
+                if (!ALL && i >= fm) break;
+                bf16x4_t ah, al;
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        short h, l;
-                        split_bf16(lds.A[buf][kk + 4 * fk + q][16 * (2 * i + wm) + fr], h, l);
-                        ah[i][q] = h;
-                        al[i][q] = l;
-                    }
-#pragma unroll
-                for (int j = 0; j < FN; ++j)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        short h, l;
-                        split_bf16(lds.B[buf][kk + 4 * fk + q][16 * (WN * j + wn) + fr], h, l);
-                        bh[j][q] = h;
-                        bl[j][q] = l;
-                    }
-#pragma unroll
-                for (int i = 0; i < FM; ++i)
-#pragma unroll
-                    for (int j = 0; j < FN; ++j)
-                        if (ALL || (i < fm && j < fn)) {
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bh[j], ah[i], acc[i][j], 0, 0, 0);
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bh[j], al[i], acc[i][j], 0, 0, 0);
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bl[j], ah[i], acc[i][j], 0, 0, 0);
-                        }
+                for (int q = 0; q < 4; ++q) {
+                    short h, l;
+                    split_bf16(lds.A[buf][4 * fk + q][16 * i + fr], h, l);
+                    ah[q] = h;
+                    al[q] = l;
+                }
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bh, ah, acc[i], 0, 0, 0);
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bh, al, acc[i], 0, 0, 0);
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bl, ah, acc[i], 0, 0, 0);
             }
         } else {
 #pragma unroll
             for (int kk = 0; kk < KS; kk += 4) {
                 if (kk < kn) {
-                    TI af[FM], bf[FN];
+                    TI af[S], bf = lds.B[buf][kk + fk][wc + fr];
 #pragma unroll
-                    for (int i = 0; i < FM; ++i) af[i] = lds.A[buf][kk + fk][16 * (2 * i + wm) + fr];
+                    for (int i = 0; i < S; ++i) af[i] = lds.A[buf][kk + fk][16 * i + fr];
 #pragma unroll
-                    for (int j = 0; j < FN; ++j) bf[j] = lds.B[buf][kk + fk][16 * (WN * j + wn) + fr];
-#pragma unroll
-                    for (int i = 0; i < FM; ++i)
-#pragma unroll
-                        for (int j = 0; j < FN; ++j)
-                            if (ALL || (i < fm && j < fn)) acc[i][j] = Mma<TI>::step(bf[j], af[i], acc[i][j]);
+                    for (int i = 0; i < S; ++i)
+                        if (ALL || i < fm) acc[i] = Mma<TI>::step(bf, af[i], acc[i]);
                 }
             }
         }
     };
-    auto reduce = [&](auto all) {
+    auto reduce = [&](auto steps, auto all) {
         int left = tile.k1 - tile.k0;
         if (left > 0) load(left);
         for (int buf = 0; left > 0; buf ^= 1, left -= KS) {
 #pragma unroll
-            for (int i = 0; i < NA; ++i) lds.A[buf][a_k(i)][a_m(i)] = ra[i];
+            for (int i = 0; i < NE; ++i) lds.A[buf][a_k(i)][a_m(i)] = ra[i];
 #pragma unroll
-            for (int i = 0; i < NB; ++i) lds.B[buf][b_k(i)][b_n(i)] = rb[i];
+            for (int i = 0; i < NE; ++i) lds.B[buf][b_k(i)][b_n(i)] = rb[i];
             __syncthreads();
             if (left > KS) load(left - KS);
-            multiply(buf, left, all);
+            if (wc < nl) multiply(buf, left, steps, all);
         }
     };
-    if (ml == BM && nl == BN) reduce(std::true_type());
-    else reduce(std::false_type());
+    if (tile.k1 <= tile.k0) __syncthreads();  // no slice: the row table still has to reach the other waves
+    if (fm == F) reduce(std::integral_constant<int, F>(), std::true_type());
+    else if (fm > 4) reduce(std::integral_constant<int, F>(), std::false_type());
+    else if (fm > 2) reduce(std::integral_constant<int, 4>(), std::false_type());
+    else reduce(std::integral_constant<int, 2>(), std::false_type());
 
     // D = C^T: register r of lane l holds C[l % 16][row(l, r)] of its 16 x 16 tile, so
     // consecutive lanes store consecutive rows of a column
+    if (wc >= nl) return;
     TO* C = static_cast<TO*>(bases.p[g.base_c]) + (rmap ? 0 : g.c + int64_t(tile.batch) * g.sc);
     const bool split = tile.ws >= 0;  // never for stacked problems
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
-        const int mm = 16 * (2 * i + wm) + fr, m = m0 + mm;
+    for (int i = 0; i < F; ++i) {
+        const int mm = 16 * i + fr, m = m0 + mm;
         if (mm >= ml) continue;
         // column n of this row at c_row + n * c_ld
         TO* c_row = C + m;
         int64_t c_ld = g.ldc;
         if (rmap) {
-            const GemmRow r = rows[g.a + m];
-            c_row = C + r.c + int64_t(tile.batch) * g.sc * r.ld;
-            c_ld = r.ld;
+            c_ld = lds.row_ld[mm];
+            c_row = C + lds.row_c[mm] + int64_t(tile.batch) * g.sc * c_ld;
         }
 #pragma unroll
-        for (int j = 0; j < FN; ++j) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int nn = 16 * (WN * j + wn) + Mma<TI>::row(lane, r);
-                if (nn >= nl) continue;
-                if (split) ws[tile.ws + mm + int64_t(nn) * BM] = acc[i][j][r];
-                else c_row[int64_t(n0 + nn) * c_ld] = TO(acc[i][j][r]);
-            }
+        for (int r = 0; r < 4; ++r) {
+            const int nn = wc + Mma<TI>::row(lane, r);
+            if (nn >= nl) continue;
+            if (split) ws[tile.ws + mm + int64_t(nn) * tile.bm] = acc[i][r];
+            else c_row[int64_t(n0 + nn) * c_ld] = TO(acc[i][r]);
         }
     }
 }
 
-template <int FM, int FN, class TI, class TO, int KS, int MINB = 1, int WN = 2, bool BF3 = false>
-__global__ __launch_bounds__(128 * WN, MINB) void gemm_kernel(const GemmDesc* __restrict__ probs,
-                                                              const GemmRow* __restrict__ rows,
-                                                              const GemmTile* __restrict__ tiles, Bases bases,
-                                                              TI* __restrict__ ws) {
-    __shared__ GemmLds<FM, FN, TI, KS, WN> lds;
-    const GemmTile tile = tiles[blockIdx.x];
+// A is transposed in FP64 only (boundary growth, the MPO-term adjoint), and never both operands
+template <class TI, class TO, bool BF3 = false>
+__global__ __launch_bounds__(GEMM_THREADS, 4) void gemm_kernel(const GemmDesc* __restrict__ probs,
+                                                               const GemmRow* __restrict__ rows,
+                                                               const GemmItem* __restrict__ items, Bases bases,
+                                                               TI* __restrict__ ws) {
+    __shared__ GemmLds<TI> lds;
+    const GemmItem tile = items[blockIdx.x];
     const GemmDesc g = probs[tile.prob];
-    const bool tb = g.flags & GEMM_TRANS_B;
-    if (g.flags & GEMM_TRANS_A) {
-        if (tb) gemm_tile<FM, FN, TI, TO, KS, WN, BF3, true, true>(lds, tile, g, rows, bases, ws);
-        else gemm_tile<FM, FN, TI, TO, KS, WN, BF3, true, false>(lds, tile, g, rows, bases, ws);
-    } else {
-        if (tb) gemm_tile<FM, FN, TI, TO, KS, WN, BF3, false, true>(lds, tile, g, rows, bases, ws);
-        else gemm_tile<FM, FN, TI, TO, KS, WN, BF3, false, false>(lds, tile, g, rows, bases, ws);
-    }
+    constexpr bool F64 = std::is_same<TI, double>::value;
+    if (g.flags & GEMM_TRANS_B) gemm_tile<TI, TO, BF3, false, true>(lds, tile, g, rows, bases, ws);
+    else if (F64 && (g.flags & GEMM_TRANS_A)) gemm_tile<TI, TO, BF3, F64, false>(lds, tile, g, rows, bases, ws);
+    else gemm_tile<TI, TO, BF3, false, false>(lds, tile, g, rows, bases, ws);
 }
 
-// C tile = sum of its split partials, added in split order; blockIdx.y selects 256 elements of
-// the tile, so one output tile is reduced by up to 64 workgroups
-constexpr int REDUCE_CHUNKS = 64;  // 16384 (largest tile) / 256
-constexpr bool reduce_covers(int sh) { return sh == GEMM_N_SHAPES || (gemm_bm(sh) * gemm_bn(sh) <= REDUCE_CHUNKS * 256 && reduce_covers(sh + 1)); }
-static_assert(reduce_covers(0), "reduce grid covers every tile shape");
+// C tile = sum of its split partials, added in split order; blockIdx.y selects 256 elements of the tile
 template <class TW, class TO>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmDesc* __restrict__ probs,
                                                           const GemmReduce* __restrict__ jobs, Bases bases,
@@ -706,66 +679,35 @@ inline unsigned grid_for(uint64_t n, int threads, unsigned cap = 8192) {
 
 namespace {
 
-// K slices of 8 with at most 128 VGPRs (two workgroups per SIMD): measured fastest for every tile
-// shape on the H*psi stages of a 24-orbital, M = 512 site problem (short and long reductions alike)
-constexpr int GEMM_KS = 8, GEMM_MINB = 4;
-
 template <class TI, class TO, bool BF3 = false>
-void launch_gemm_t(const GemmDesc* probs, const GemmRow* rows, const GemmTile* const* tiles, const int64_t* n_tiles,
-                   const GemmReduce* reduces, int64_t n_reduces, void* ws, Bases bases, hipStream_t stream) {
+void launch_gemm_t(const GemmDesc* probs, const GemmRow* rows, const GemmItem* items, int64_t n_items,
+                   const GemmReduce* reduces, int64_t n_reduces, int32_t reduce_elems, void* ws, Bases bases,
+                   hipStream_t stream) {
     TI* w = static_cast<TI*>(ws);
-    constexpr int KSL = BF3 ? 16 : GEMM_KS;  // split-BF16 steps take 16 k at a time
-    for (int sh = 0; sh < GEMM_N_SHAPES; ++sh) {
-        for (int64_t off = 0; off < n_tiles[sh]; off += 0x7fffffff) {
-            int64_t cnt = n_tiles[sh] - off < 0x7fffffff ? n_tiles[sh] - off : 0x7fffffff;
-            if (sh == GEMM_32x128)
-                hipLaunchKernelGGL((gemm_kernel<1, 4, TI, TO, KSL, GEMM_MINB, 2, BF3>), dim3(unsigned(cnt)), dim3(256), 0, stream, probs,
-                                   rows, tiles[sh] + off, bases, w);
-            else if (sh == GEMM_64x64)
-                hipLaunchKernelGGL((gemm_kernel<2, 2, TI, TO, KSL, GEMM_MINB, 2, BF3>), dim3(unsigned(cnt)), dim3(256), 0, stream, probs,
-                                   rows, tiles[sh] + off, bases, w);
-            else if (sh == GEMM_96x64)
-                hipLaunchKernelGGL((gemm_kernel<3, 2, TI, TO, KSL, GEMM_MINB, 2, BF3>), dim3(unsigned(cnt)), dim3(256), 0, stream, probs,
-                                   rows, tiles[sh] + off, bases, w);
-            else if (sh == GEMM_64x128)
-                hipLaunchKernelGGL((gemm_kernel<2, 4, TI, TO, KSL, GEMM_MINB, 2, BF3>), dim3(unsigned(cnt)), dim3(256), 0, stream, probs,
-                                   rows, tiles[sh] + off, bases, w);
-            else if (sh == GEMM_128x128)
-                hipLaunchKernelGGL((gemm_kernel<4, 2, TI, TO, KSL, GEMM_MINB / 2, 4, BF3>), dim3(unsigned(cnt)), dim3(512), 0,
-                                   stream, probs, rows, tiles[sh] + off, bases, w);
-            else
-                hipLaunchKernelGGL((gemm_kernel<4, 2, TI, TO, KSL, GEMM_MINB, 2, BF3>), dim3(unsigned(cnt)), dim3(256), 0, stream, probs,
-                                   rows, tiles[sh] + off, bases, w);
-        }
+    for (int64_t off = 0; off < n_items; off += 0x7fffffff) {
+        const int64_t cnt = n_items - off < 0x7fffffff ? n_items - off : 0x7fffffff;
+        hipLaunchKernelGGL((gemm_kernel<TI, TO, BF3>), dim3(unsigned(cnt)), dim3(GEMM_THREADS), 0, stream, probs, rows,
+                           items + off, bases, w);
     }
     for (int64_t off = 0; off < n_reduces; off += 0x7fffffff) {
-        int64_t cnt = n_reduces - off < 0x7fffffff ? n_reduces - off : 0x7fffffff;
-        hipLaunchKernelGGL((gemm_reduce_kernel<TI, TO>), dim3(unsigned(cnt), REDUCE_CHUNKS), dim3(256), 0, stream,
-                           probs, reduces + off, bases, w);
+        const int64_t cnt = n_reduces - off < 0x7fffffff ? n_reduces - off : 0x7fffffff;
+        hipLaunchKernelGGL((gemm_reduce_kernel<TI, TO>), dim3(unsigned(cnt), unsigned((reduce_elems + 255) / 256)), dim3(256),
+                           0, stream, probs, reduces + off, bases, w);
     }
 }
 
 }  // namespace
 
-hipError_t launch_gemm(GemmPrec prec, const GemmDesc* probs, const GemmRow* rows, const GemmTile* const* tiles,
-                       const int64_t* n_tiles, const GemmReduce* reduces, int64_t n_reduces, void* ws, Bases bases,
+hipError_t launch_gemm(GemmPrec prec, const GemmDesc* probs, const GemmRow* rows, const GemmItem* items, int64_t n_items,
+                       const GemmReduce* reduces, int64_t n_reduces, int32_t reduce_elems, void* ws, Bases bases,
                        hipStream_t stream) {
+    auto run = [&](auto launch) { launch(probs, rows, items, n_items, reduces, n_reduces, reduce_elems, ws, bases, stream); };
     switch (prec) {
-        case GEMM_F64:
-            launch_gemm_t<double, double>(probs, rows, tiles, n_tiles, reduces, n_reduces, ws, bases, stream);
-            break;
-        case GEMM_F32:
-            launch_gemm_t<float, float>(probs, rows, tiles, n_tiles, reduces, n_reduces, ws, bases, stream);
-            break;
-        case GEMM_F32_OUT_F64:
-            launch_gemm_t<float, double>(probs, rows, tiles, n_tiles, reduces, n_reduces, ws, bases, stream);
-            break;
-        case GEMM_BF3:
-            launch_gemm_t<float, float, true>(probs, rows, tiles, n_tiles, reduces, n_reduces, ws, bases, stream);
-            break;
-        case GEMM_BF3_OUT_F64:
-            launch_gemm_t<float, double, true>(probs, rows, tiles, n_tiles, reduces, n_reduces, ws, bases, stream);
-            break;
+        case GEMM_F64: run(launch_gemm_t<double, double>); break;
+        case GEMM_F32: run(launch_gemm_t<float, float>); break;
+        case GEMM_F32_OUT_F64: run(launch_gemm_t<float, double>); break;
+        case GEMM_BF3: run(launch_gemm_t<float, float, true>); break;
+        case GEMM_BF3_OUT_F64: run(launch_gemm_t<float, double, true>); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

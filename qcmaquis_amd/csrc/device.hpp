@@ -21,11 +21,11 @@ struct Bases {
 // GEMM_BF3*: FP32 operands, split-BF16 products (hi hi + hi lo + lo hi) on the BF16 matrix cores
 enum GemmPrec { GEMM_F64 = 0, GEMM_F32 = 1, GEMM_F32_OUT_F64 = 2, GEMM_BF3 = 3, GEMM_BF3_OUT_F64 = 4 };
 
-// grouped GEMM stage: tiles of each shape (GemmShape) then the split-K reduce jobs; ws is the
-// workspace of the split partials (GemmSchedule::ws_elems elements of the compute type); rows is
-// the row table of the stage's stacked (GEMM_ROWMAP) problems
-hipError_t launch_gemm(GemmPrec prec, const GemmDesc* probs, const GemmRow* rows, const GemmTile* const* tiles,
-                       const int64_t* n_tiles, const GemmReduce* reduces, int64_t n_reduces, void* ws, Bases bases,
+// grouped GEMM stage: its work items, then the split-K reduce jobs (of tiles of at most reduce_elems
+// elements); ws is the workspace of the split partials (GemmSchedule::ws_elems elements of the
+// compute type); rows is the row table of the stage's stacked (GEMM_ROWMAP) problems
+hipError_t launch_gemm(GemmPrec prec, const GemmDesc* probs, const GemmRow* rows, const GemmItem* items, int64_t n_items,
+                       const GemmReduce* reduces, int64_t n_reduces, int32_t reduce_elems, void* ws, Bases bases,
                        hipStream_t stream);
 // block-form MPO-term sum (SBlockTable uploaded; alpha, T and S of type T): writes every S tile
 // of the table's lines; xcd_contiguous: each XCD takes a contiguous range of the work list

@@ -1820,12 +1820,12 @@ GemmPolicy gemm_policy(int i) {
     require(i >= 0 && i < GEMM_N_POLICIES, "gemm policy: index out of range");
     GemmPolicy p;
     switch (i) {
-        case 1: p.wide = 1; break;              // 64- and 128-column tiles only by M
-        case 2: p.wide = 2; break;              // 128-column tiles whenever N > 64
-        case 3: p.tiles96 = 0; break;           // 128-row tiles from 65 rows
-        case 4: p.target_items = 8192; break;   // split along K more readily
-        case 5: p.target_items = 2048; break;   // split along K less
-        case 6: p.min_chunk = 512; break;       // longer K ranges per split tile
+        case 1: p.target_items = 1024; break;   // split along K less
+        case 2: p.target_items = 2048; break;
+        case 3: p.target_items = 8192; break;   // split along K more readily
+        case 4: p.min_chunk = 512; break;       // longer K ranges per split tile
+        case 5: p.target_items = 8192; p.min_chunk = 128; break;
+        case 6: p.target_items = 2048; p.min_chunk = 512; break;
         default: break;
     }
     return p;
@@ -1867,39 +1867,19 @@ GemmSchedule build_gemm_schedule(std::vector<GemmDesc> const& probs, GemmPolicy 
     const int64_t target_items = pol.target_items;
     const int32_t min_chunk = pol.min_chunk;
     require(min_chunk >= 16 && min_chunk % 16 == 0, "gemm schedule: chunk must be a multiple of 16");
-    require(pol.wide >= 0 && pol.wide <= 2, "gemm schedule: wide mode 0, 1 or 2");
     GemmSchedule S;
-    // 96-row tiles (for 64 < M <= 96) only for problems with a plain A operand: a stacked problem's
-    // threads each load one row, which needs a tile height that divides 256.  64x128 tiles (for
-    // 32 < M <= 64, N > 64) only when the stage has too few tiles to fill the device and is split
-    // along K anyway: then the wider tile halves the A re-reads at no cost in parallelism
-    bool wide = pol.wide == 2;
-    auto shape_of = [&](GemmDesc const& g) {
-        const bool w = wide && g.N > 64 && !(g.flags & GEMM_ROWMAP);
-        return g.M <= 32 ? GEMM_32x128
-             : g.M <= 64 ? ((wide && g.N > 64) ? GEMM_64x128 : GEMM_64x64)
-             : (pol.tiles96 && g.M <= 96 && !(g.flags & GEMM_ROWMAP)) ? GEMM_96x64
-             : w ? GEMM_128x128 : GEMM_128x64;
-    };
-    auto tiles_of = [&](GemmDesc const& g) {
-        int sh = shape_of(g);
-        return int64_t((g.M + gemm_bm(sh) - 1) / gemm_bm(sh)) * ((g.N + gemm_bn(sh) - 1) / gemm_bn(sh)) * g.batch;
-    };
-    auto count = [&](int64_t& n_tiles, double& work) {
-        n_tiles = 0;
-        work = 0;
-        for (auto const& g : probs) {
-            if (g.M <= 0 || g.N <= 0) continue;
-            n_tiles += tiles_of(g);
-            work += double(tiles_of(g)) * g.K;
-        }
+    auto shape_of = [](GemmDesc const& g) {
+        const int32_t nt = (g.M + 127) / 128, h = (g.M + nt - 1) / nt;
+        return h <= 32 ? GEMM_32 : h <= 64 ? GEMM_64 : h <= 96 ? GEMM_96 : GEMM_128;
     };
     int64_t n_tiles = 0;
     double work = 0;
-    count(n_tiles, work);
-    if (n_tiles < target_items && target_items > 0 && pol.wide == 0) {
-        wide = true;
-        count(n_tiles, work);
+    for (auto const& g : probs) {
+        if (g.M <= 0 || g.N <= 0) continue;
+        const int sh = shape_of(g);
+        const int64_t n = int64_t((g.M + gemm_bm(sh) - 1) / gemm_bm(sh)) * ((g.N + gemm_bn(sh) - 1) / gemm_bn(sh)) * g.batch;
+        n_tiles += n;
+        work += double(n) * g.K;
     }
     // K range per workgroup when the stage alone cannot fill the device
     int64_t chunk = INT64_MAX;
@@ -1939,6 +1919,21 @@ GemmSchedule build_gemm_schedule(std::vector<GemmDesc> const& probs, GemmPolicy 
     for (auto& v : S.tiles)
         std::stable_sort(v.begin(), v.end(), [](GemmTile const& a, GemmTile const& b) { return a.k1 - a.k0 > b.k1 - b.k0; });
     return S;
+}
+
+std::vector<GemmItem> gemm_items(std::vector<GemmDesc> const& probs, GemmSchedule const& sch) {
+    std::vector<GemmItem> out;
+    out.reserve(size_t(sch.n_tiles()));
+    for (int sh = 0; sh < GEMM_N_SHAPES; ++sh) {
+        const int32_t bm = gemm_bm(sh), bn = gemm_bn(sh);
+        for (GemmTile const& t : sch.tiles[sh])
+            out.push_back(GemmItem{t.prob, t.batch, t.tm * bm, std::min(bm, probs[size_t(t.prob)].M - t.tm * bm), t.tn * bn,
+                                   t.k0, t.k1, bm, t.ws});
+    }
+    std::stable_sort(out.begin(), out.end(), [](GemmItem const& a, GemmItem const& b) {
+        return int64_t(a.k1 - a.k0) * a.bm > int64_t(b.k1 - b.k0) * b.bm;
+    });
+    return out;
 }
 
 // ---- host-side bounds validation of every device table (a table entry that would leave its

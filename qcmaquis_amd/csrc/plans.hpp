@@ -181,28 +181,14 @@ constexpr int SBLOCK_ELEMS = 128;
 // the block term sum loads one element past a tile of odd size: T buffers are that much longer
 constexpr int SB_T_SPARE = 2;
 
-// Execution schedule of a grouped GEMM stage.  Output tiles come in six shapes (BM x BN):
-// 32x128 for M <= 32, 64x64 for M <= 64, 96x64 for M <= 96 (problems without a row table), 128x64
-// above; in a stage that is split along K (fewer output tiles than the device takes) problems
-// with N > 64 take the 128-column tiles 64x128 and (M > 96, without a row table) 128x128, so the A
-// panel is read once per 128 output columns (128x128 on eight waves).  So a
-// problem with a short M edge is not padded to a taller tile and the B panel of a tall problem is
-// read once.  When the stage has too few
-// tiles to fill the device, long reductions are split along K: each split tile writes its
-// partial BM x BN tile (column-major, ld BM) into a workspace and a reduce job adds the
-// partials in split order into C, so the result does not depend on scheduling.
-enum GemmShape {
-    GEMM_32x128 = 0, GEMM_64x64 = 1, GEMM_128x64 = 2, GEMM_96x64 = 3, GEMM_64x128 = 4, GEMM_128x128 = 5,
-    GEMM_N_SHAPES = 6
-};
-constexpr int gemm_bm(int shape) {
-    return shape == GEMM_32x128 ? 32
-         : (shape == GEMM_64x64 || shape == GEMM_64x128) ? 64
-         : shape == GEMM_96x64 ? 96 : 128;
-}
-constexpr int gemm_bn(int shape) {
-    return (shape == GEMM_32x128 || shape == GEMM_64x128 || shape == GEMM_128x128) ? 128 : 64;
-}
+// Execution schedule of a grouped GEMM stage.  Output tiles are 128 columns wide and 32, 64, 96 or 128
+// rows tall: a problem's rows are cut into the fewest tiles of at most 128 rows, of about equal
+// height.  When the stage has too few tiles to fill the device, long reductions are split along K:
+// each split tile writes its partial BM x BN tile (column-major, ld BM) into a workspace and a
+// reduce job adds the partials in split order into C, so the result does not depend on scheduling.
+enum GemmShape { GEMM_32 = 0, GEMM_64, GEMM_96, GEMM_128, GEMM_N_SHAPES };
+constexpr int gemm_bm(int shape) { return 32 * (shape + 1); }
+constexpr int gemm_bn(int) { return 128; }
 struct GemmTile {
     int32_t prob, batch, tm, tn;
     int32_t k0, k1;   // reduction range of this tile
@@ -225,14 +211,13 @@ struct GemmSchedule {
         return n;
     }
 };
-// The choices of a grouped GEMM schedule that the tile autotuner varies.  wide: 0 = 128-column
-// tiles (64x128, 128x128) for N > 64 when the stage is split along K, 1 = never, 2 = always;
-// tiles96: 96-row tiles for 64 < M <= 96 (problems without a row table), else 128 rows;
-// target_items: workgroups a stage should provide before K is split; min_chunk: shortest K range
-// of a split tile (a multiple of the K step 16)
+// The choices of a grouped GEMM schedule that the tile autotuner varies.  target_items: workgroups
+// a stage should provide before K is split; min_chunk: shortest K range of a split tile (a multiple
+// of the K step 16).  L*S stages in us at targets
+// of 2048 / 4096: 18 orbitals and M = 509 376 / 400, 20 with spins and M = 700 865 / 901, M = 2048
+// 15.5 / 15.1 ms (17.1 at 1024); the shorter ranges of 4096 keep the FP32 rounding down (18 orbitals,
+// M = 512: 4.3e-7 at 2048, 3.5e-7 at 4096)
 struct GemmPolicy {
-    int32_t wide = 0;
-    int32_t tiles96 = 1;
     int64_t target_items = 4096;
     int32_t min_chunk = 256;
 };
@@ -247,6 +232,19 @@ inline GemmSchedule build_gemm_schedule(std::vector<GemmDesc> const& probs, int6
     p.min_chunk = min_chunk;
     return build_gemm_schedule(probs, p);
 }
+// Work item of the device's GEMM kernel: rows [m0, m0 + ml), ml <= 128, and up to 128 columns from n0 of
+// a problem's C (of batch entry `batch`), reduced over [k0, k1); ws < 0: written to C, else the
+// partial tile at element ws of the workspace with leading dimension bm.
+struct GemmItem {
+    int32_t prob, batch;
+    int32_t m0, ml, n0;
+    int32_t k0, k1;
+    int32_t bm;
+    int64_t ws;
+};
+static_assert(sizeof(GemmItem) == 40, "GemmItem layout");
+// the work items of a schedule, all shapes in one list, the most work first
+std::vector<GemmItem> gemm_items(std::vector<GemmDesc> const& probs, GemmSchedule const& sch);
 // Key of a stage's (m, n, k) histogram for the autotuner: the flop-weighted means of log2 M,
 // log2 N and log2 K (in quarters), the share of flops in problems of at most 32, 64 and 96 rows
 // (in eighths), log2 of the output tiles at the default rule, and whether rows come from a row

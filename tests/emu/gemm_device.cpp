@@ -1,7 +1,10 @@
-// Host-side check of the device form of a grouped GEMM stage -- test code: the operand and output
-// addresses of every element of the folded T-GEMMs equal those of the plan's own problems.
+// Host-side checks of the device form of a grouped GEMM stage -- test code: the operand and output
+// addresses of every element of the folded T-GEMMs equal those of the plan's own problems, and the
+// work items of a schedule cover every element of C and of its reduction once.
+#include <algorithm>
 #include <cstdio>
 #include <stdexcept>
+#include <vector>
 
 #include "descriptors.hpp"
 #include "plans.hpp"
@@ -44,6 +47,52 @@ extern "C" long fold_check(int sym, const mq_mpo_desc* md, const mq_bindex_desc*
         return folded;
     } catch (std::exception const& e) {
         fprintf(stderr, "fold_check: %s\n", e.what());
+        return -1;
+    }
+}
+
+// work items of C problems of the given sizes under schedule candidate `policy`; splits or -1
+extern "C" long items_check(int n, const int* M, const int* N, const int* K, int batch, int policy) {
+    try {
+        std::vector<GemmDesc> G;
+        for (int i = 0; i < n; ++i) {
+            GemmDesc g{};
+            g.M = M[i];
+            g.N = N[i];
+            g.K = K[i];
+            g.batch = batch;
+            G.push_back(g);
+        }
+        const GemmSchedule sch = build_gemm_schedule(G, gemm_policy(policy));
+        std::vector<std::vector<int64_t>> done(size_t(n) * batch);
+        for (int i = 0; i < n; ++i)
+            for (int b = 0; b < batch; ++b) done[size_t(i) * batch + b].assign(size_t(M[i]) * N[i], 0);
+        std::vector<char> ws(sch.ws_elems, 0);
+        long splits = 0;
+        for (GemmItem const& t : gemm_items(G, sch)) {
+            GemmDesc const& g = G.at(size_t(t.prob));
+            const int nl = std::min(128, g.N - t.n0);
+            require(t.ml > 0 && t.ml <= t.bm && t.bm <= 128 && t.m0 + t.ml <= g.M && nl > 0, "items: shape");
+            require(t.k0 >= 0 && t.k0 < t.k1 && t.k1 <= g.K && t.k0 % 16 == 0, "items: K range");
+            require(t.ws >= 0 || t.k1 - t.k0 == g.K, "items: split without a partial");
+            auto& d = done[size_t(t.prob) * batch + t.batch];
+            for (int c = 0; c < nl; ++c)
+                for (int r = 0; r < t.ml; ++r) {
+                    d[size_t(t.m0 + r) + size_t(t.n0 + c) * g.M] += t.k1 - t.k0;
+                    if (t.ws >= 0) {
+                        char& w = ws.at(size_t(t.ws + r + int64_t(c) * t.bm));
+                        require(!w, "items: partials overlap");
+                        w = 1;
+                    }
+                }
+            splits += t.ws >= 0;
+        }
+        for (int i = 0; i < n; ++i)
+            for (int b = 0; b < batch; ++b)
+                for (int64_t v : done[size_t(i) * batch + b]) require(v == K[i], "items: cover");
+        return splits;
+    } catch (std::exception const& e) {
+        fprintf(stderr, "items_check: %s\n", e.what());
         return -1;
     }
 }

@@ -24,6 +24,9 @@ def lib():
     lib.fold_check.restype = C.c_long
     lib.fold_check.argtypes = [C.c_int, C.POINTER(abi.MPODesc), C.POINTER(abi.BIndexDesc), C.POINTER(abi.BIndexDesc), idx,
                                idx, idx]
+    ints = C.POINTER(C.c_int)
+    lib.items_check.restype = C.c_long
+    lib.items_check.argtypes = [C.c_int, ints, ints, ints, C.c_int, C.c_int]
     return lib
 
 
@@ -48,3 +51,13 @@ def test_folded_batches(oracle_lib, lib):
             assert f >= 0, (sym, seed, k)
             folded += f
     assert folded > 0
+
+
+@pytest.mark.parametrize("policy", range(7))
+def test_work_items(lib, policy):
+    """tiles, K splits and partials over sizes around the tile heights, widths and K steps"""
+    m = [1, 15, 32, 33, 64, 96, 97, 128, 129, 200, 257, 300]
+    n = [1, 16, 127, 128, 129, 300, 5, 40, 260, 64, 33, 130]
+    k = [1, 17, 256, 1000, 513, 3, 16, 700, 2049, 128, 4000, 31]
+    arr = [(C.c_int * len(v))(*v) for v in (m, n, k)]
+    assert lib.items_check(len(m), *arr, 2, policy) > 0
