@@ -65,7 +65,8 @@ extern "C" {
                                   tiles of at most this many elements term by term, one lane per
                                   element, instead of in 16-tile blocks on the matrix cores (0: every
                                   tile in blocks); MQ_SMALL_TILE_AUTO (default): per site problem,
-                                  64 when its mean S tile has at most 16 elements, else 0 */
+                                  64 when its mean S tile has at most 16 elements and the plan at
+                                  most 2^19 terms, else 0 */
 #define MQ_SMALL_TILE_AUTO (-1)
 #define MQ_OPT_CHUNK_MB 3      /* value >= 0: H*psi plans made afterwards split their output columns
                                   by right sector into chunks of at most this many MiB of FP64 T and

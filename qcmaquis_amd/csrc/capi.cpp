@@ -1052,7 +1052,7 @@ static void finish_plan(mq_ctx_t ctx, mq_hpsi_plan_s* p, std::vector<LpanelPart>
     for (size_t i = 0; i + 1 < line_ranges.size(); ++i) {
         const size_t l0 = line_ranges[i], l1 = line_ranges[i + 1];
         mark_small_lines(H.lines, l0, l1, ctx->small_tile_max == MQ_SMALL_TILE_AUTO
-                                              ? auto_small_tile_max(H.lines, l0, l1) : ctx->small_tile_max);
+                                              ? auto_small_tile_max(H.lines, l0, l1, H.terms.size()) : ctx->small_tile_max);
     }
     // per chunk: its GEMM problems (T-GEMM rows re-based on the chunk's row table), checked against
     // the chunk's T and S sizes, their schedules, and the term-sum block tables of its lines

@@ -301,7 +301,8 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmDesc* __rest
 // tile offsets go to LDS without passing through registers.  The waves of a workgroup work by the
 // block's tile size (SWorkCounts): one block on all of them (SBLOCK_ELEMS elements, tables staged
 // once per workgroup), a block of 33 to 64 elements on two, or one block per wave; in the last two
-// every wave stages its own block's tables and runs without barriers.
+// every wave stages its own block's tables and runs without barriers.  A block of at most 64 elements
+// with many k-steps (SB_SHARE) has them shared out over the workgroup, the sums meeting in LDS.
 //
 // Bound: L2-miss traffic (every block reads the union of its T tiles, T 2.1-2.5 times in all, and
 // writes S) where tiles are large, waiting on the chain tables -> tiles -> matrix cores where they
@@ -361,18 +362,25 @@ __global__ __launch_bounds__(SB_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     SWork w = launch[wg];
     const bool team = w.blk >= 0;
-    int sub = wave;  // this wave's slice of its work item
-    if (!team) {     // -w.blk waves per item, from work[w.n0]
-        const int lw = -w.blk - 1, wi = w.n0 + (wave >> lw);
+    int sub = wave;              // this wave's slice of its work item
+    int part = 0, parts = 1;     // its share of the k-steps
+    if (!team) {                 // item work[w.n0] and, unless its k-steps are shared, the next ones
+        const bool shared = w.blk < -2;
+        const int lw = (-w.blk - 1) & 1, wi = w.n0 + (shared ? 0 : wave >> lw);
         sub = wave & lw;
+        if (shared) {
+            part = wave >> lw;
+            parts = SB_WAVES >> lw;
+        }
         if (wi >= (lw ? n.team + n.pair : n.team + n.pair + n.solo)) return;
         w = work[wi];
     }
     const SBlock b = blocks[w.blk];
+    const int k0 = b.nk * part / parts, k1 = b.nk * (part + 1) / parts;
     const int n0 = w.n0 + 16 * SB_NC * sub;
     // a wave past the tile end loads and stores no tile but takes part in its team's barriers
     const bool active = n0 < b.E;
-    if (!team && !active) return;
+    if (!team && !active) return;  // never where k-steps are shared: those tiles fill their waves
     const int li = lane & 15, lk = lane >> 4;
     T* al = s_alpha + (team ? 0 : wave * SB_SUB1 * 64);
     int64_t* of = s_off + (team ? 0 : wave * SB_KS1 * 4);
@@ -393,13 +401,13 @@ __global__ __launch_bounds__(SB_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 
     lds_fetch(lsoff + b.line0, so, SBLOCK_LINES * 8, st_lane, st_lanes);
     lds_fetch(llds + b.line0, ld, SBLOCK_LINES * 4, st_lane, st_lanes);
-    for (int c0 = 0; c0 < b.nk;) {
+    for (int c0 = k0; c0 < k1;) {
         // the next k-steps whose tables fit: lane l looks at k-step c0 + l
         const int kl = c0 + lane;
-        const uint32_t word = kl < b.nk ? kw[kl] : 0;
+        const uint32_t word = kl < k1 ? kw[kl] : 0;
         const int a0 = __builtin_amdgcn_readfirstlane(int(word >> 8));
         const int end = kl + 1 < b.nk ? int(kw[kl + 1] >> 8) : b.na;
-        const int cn = __builtin_popcountll(__ballot(kl < b.nk && lane < cap_k && end - a0 <= cap_sub));
+        const int cn = __builtin_popcountll(__ballot(kl < k1 && lane < cap_k && end - a0 <= cap_sub));
         const int an = __builtin_amdgcn_readlane(end, cn - 1) - a0;
         if (team && c0 > 0) __syncthreads();  // the previous k-steps' tables are consumed
         asm volatile("" ::: "memory");
@@ -445,10 +453,31 @@ __global__ __launch_bounds__(SB_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
         }
         c0 += cn;
     }
-    if (b.nk == 0) {
+    if (k0 == k1) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (team) __syncthreads();
     }
+    // shared k-steps: the upper half of the parts hands its sums to the lower half until one is left
+    for (int h = parts / 2; h > 0; h /= 2) {
+        constexpr int NV = SBLOCK_GROUPS * SB_NC * 4;
+        static_assert(SB_WAVES / 2 * NV <= SB_SUB, "the sums of half the waves fit the coefficient buffer");
+        T* p = s_alpha + 64 * NV * ((part % h) * (SB_WAVES / parts) + sub) + lane;
+        __syncthreads();
+        if (part >= h && part < 2 * h)
+#pragma unroll
+            for (int g = 0; g < SBLOCK_GROUPS; ++g)
+                if (SBLOCK_GROUP * g < b.nlines)
+#pragma unroll
+                    for (int v = 0; v < SB_NC * 4; ++v) p[64 * (SB_NC * 4 * g + v)] = acc[g][v / 4][v % 4];
+        __syncthreads();
+        if (part < h)
+#pragma unroll
+            for (int g = 0; g < SBLOCK_GROUPS; ++g)
+                if (SBLOCK_GROUP * g < b.nlines)
+#pragma unroll
+                    for (int v = 0; v < SB_NC * 4; ++v) acc[g][v / 4][v % 4] += p[64 * (SB_NC * 4 * g + v)];
+    }
+    if (part > 0) return;
     if (!active || e0 >= b.E) return;
     // register r of lane l holds Y_g[line row(l, r)][element]: the lane's elements are stored at once
     // unless a tile column ends among them
@@ -473,33 +502,56 @@ __global__ __launch_bounds__(SB_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
         }
 }
 
-// Small-tile MPO-term sum: a work item is up to 256 >> lg lines of 2^lg lanes each (tile elements
-// <= 2^lg); lane e of a line sums alpha_k * T[t_off_k + e] over the line's terms in term order,
-// four terms' loads ahead of their multiply-adds, and writes element e of the line's S tile.  The
-// lanes of a line read the same term entries; no LDS and no barrier, so lanes past their line's
-// tile simply return.
+// Small-tile MPO-term sum: a work item is up to 256 >> (lg + ts) lines of 2^ts shares of 2^lg lanes
+// (tile elements <= 2^lg); lane e of share s sums alpha_k * T[t_off_k + e] over the line's terms
+// k = s, s + 2^ts, ..., four at a time, the shares are added by lane exchanges (between waves: through
+// LDS), and element e of the line's S tile is written once.  Past its last term a lane reads that
+// term again and leaves it out.
+//
+// Bound: the chain terms -> tile elements in the few, small problems that come here (most lines have
+// one or two terms, the longest hundreds).  One lane per element for all of a line's terms, as
+// before, took 24 us for 8 orbitals and M = 40; with a line's terms shared out 10.5.
 template <class T>
 __global__ __launch_bounds__(SMALL_LINE_LANES) void small_lines_kernel(const SSmallWork* __restrict__ work,
                                                                        const SLine* __restrict__ lines,
                                                                        const STerm* __restrict__ terms,
                                                                        const T* __restrict__ X, T* __restrict__ S) {
+    __shared__ T part[SMALL_LINE_LANES];
     const SSmallWork w = work[blockIdx.x];
-    const int li = int(threadIdx.x) >> w.lg, e = int(threadIdx.x) & ((1 << w.lg) - 1);
-    if (li >= w.n) return;
-    const SLine l = lines[w.line0 + li];
-    if (e >= l.rows * l.cols) return;
+    const int W = 1 << (w.lg + w.ts), G = 1 << w.lg;  // lanes of a line, of a share
+    const int tid = int(threadIdx.x), li = tid >> (w.lg + w.ts), q = tid & (W - 1), e = q & (G - 1);
+    const SLine l = lines[w.line0 + (li < w.n ? li : 0)];
+    const bool in = li < w.n && e < l.rows * l.cols;
     T acc = T(0);
-    int k = l.t0;
-    for (; k + 4 <= l.t1; k += 4) {
-        const STerm a = terms[k], b = terms[k + 1], c = terms[k + 2], d = terms[k + 3];
-        const T xa = X[a.t_off + e], xb = X[b.t_off + e], xc = X[c.t_off + e], xd = X[d.t_off + e];
-        acc += T(a.alpha) * xa;
-        acc += T(b.alpha) * xb;
-        acc += T(c.alpha) * xc;
-        acc += T(d.alpha) * xd;
+    if (in) {
+        constexpr int U = SMALL_LINE_DEPTH;
+        const int last = l.t1 - 1;
+        for (int k = l.t0 + (q >> w.lg); k < l.t1; k += U << w.ts) {
+            STerm t[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int ku = k + (u << w.ts);
+                t[u] = terms[ku < last ? ku : last];
+            }
+            T x[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) x[u] = X[t[u].t_off + e];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const bool ok = k + (u << w.ts) <= last;
+                acc += ok ? T(t[u].alpha) * x[u] : T(0);
+            }
+        }
     }
-    for (; k < l.t1; ++k) acc += T(terms[k].alpha) * X[terms[k].t_off + e];
-    S[l.s_off + e % l.rows + int64_t(e / l.rows) * l.lds] = acc;
+    for (int off = G; off < (W < 64 ? W : 64); off *= 2) acc += __shfl_xor(acc, off);
+    if (W > 64) {
+        part[tid] = acc;
+        __syncthreads();
+        const int step = G > 64 ? G : 64;
+        if (q < G)
+            for (int off = step; off < W; off += step) acc += part[tid + off];
+    }
+    if (in && q < G) S[l.s_off + e % l.rows + int64_t(e / l.rows) * l.lds] = acc;
 }
 
 // One S line (rows x cols tile at s_off, leading dimension lds) per workgroup; element e of the

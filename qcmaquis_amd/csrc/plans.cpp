@@ -1375,12 +1375,12 @@ GrowPlanHost build_rstep_plan(Sym sym, MPO const& mpo, BoundaryIndex const& R, M
 }
 
 // ---- block form of the MPO-term sum ------------------------------------------------------------
-// small-tile lines: ordered by lanes per line (the power of two >= rows * cols), then by term
-// count (longest first), with their terms copied in that order
+// small-tile lines: those with the most shares of their terms first, then by lanes per share (the
+// power of two >= rows * cols), neighbours staying together, with their terms copied in that order
 template <class Pred>
 static void build_small_lines(SBlockTable& B, HostTable<SLine> const& lines, HostTable<STerm> const& terms,
                               Pred is_small) {
-    struct Key { int32_t lg, nt; uint32_t i; };
+    struct Key { int32_t lg, ts, nt; uint32_t i; };
     std::vector<Key> keys;
     for (uint32_t i = 0; i < lines.size(); ++i) {
         SLine const& l = lines[i];
@@ -1388,10 +1388,13 @@ static void build_small_lines(SBlockTable& B, HostTable<SLine> const& lines, Hos
         require(int64_t(l.rows) * l.cols <= SMALL_LINE_LANES, "S blocks: small-tile line wider than 256 elements");
         int32_t lg = 0;
         while ((1 << lg) < l.rows * l.cols) ++lg;
-        keys.push_back(Key{lg, l.t1 - l.t0, i});
+        const int32_t nt = l.t1 - l.t0;
+        int32_t ts = 0;
+        while ((1 << (lg + ts)) < SMALL_LINE_LANES && nt > (SMALL_LINE_DEPTH << ts)) ++ts;
+        keys.push_back(Key{lg, ts, nt, i});
     }
     std::stable_sort(keys.begin(), keys.end(), [](Key const& a, Key const& b) {
-        return a.lg != b.lg ? a.lg < b.lg : a.nt > b.nt;
+        return a.ts != b.ts ? a.ts > b.ts : a.lg < b.lg;
     });
     std::vector<int64_t> t_start(keys.size() + 1, 0);
     for (size_t q = 0; q < keys.size(); ++q) t_start[q + 1] = t_start[q] + keys[q].nt;
@@ -1407,19 +1410,22 @@ static void build_small_lines(SBlockTable& B, HostTable<SLine> const& lines, Hos
         B.small_lines[size_t(q)] = l;
     }
     for (size_t q = 0; q < keys.size();) {
-        const int32_t lg = keys[q].lg, per = SMALL_LINE_LANES >> lg;
+        const int32_t lg = keys[q].lg, ts = keys[q].ts, per = SMALL_LINE_LANES >> (lg + ts);
         int32_t n = 0;
-        while (q + size_t(n) < keys.size() && keys[q + size_t(n)].lg == lg && n < per) ++n;
-        B.small_work.push_back(SSmallWork{int32_t(q), n, lg, 0});
+        while (q + size_t(n) < keys.size() && keys[q + size_t(n)].lg == lg && keys[q + size_t(n)].ts == ts && n < per) ++n;
+        B.small_work.push_back(SSmallWork{int32_t(q), n, lg, ts});
         q += size_t(n);
     }
     for (SLine const& l : B.small_lines) B.small_gathered += uint64_t(l.t1 - l.t0) * uint64_t(l.rows) * l.cols;
 }
 
-int32_t auto_small_tile_max(HostTable<SLine> const& lines, size_t l0, size_t l1) {
-    uint64_t e = 0;
-    for (size_t i = l0; i < l1; ++i) e += uint64_t(lines[i].rows) * uint64_t(lines[i].cols);
-    return l1 > l0 && e <= 16 * uint64_t(l1 - l0) ? 64 : 0;
+int32_t auto_small_tile_max(HostTable<SLine> const& lines, size_t l0, size_t l1, uint64_t n_terms) {
+    uint64_t e = 0, t = 0;
+    for (size_t i = l0; i < l1; ++i) {
+        e += uint64_t(lines[i].rows) * uint64_t(lines[i].cols);
+        t += uint64_t(lines[i].t1 - lines[i].t0);
+    }
+    return l1 > l0 && e <= 16 * uint64_t(l1 - l0) && std::max(t, n_terms) <= SMALL_TERMS_MAX ? 64 : 0;
 }
 
 void mark_small_lines(HostTable<SLine>& lines, size_t l0, size_t l1, int32_t limit) {
@@ -1627,8 +1633,14 @@ SBlockTable build_sblocks(HostTable<SLine> const& lines, HostTable<STerm> const&
     {
         const int64_t nt = B.n_work.team, np = B.n_work.pair, ns = B.n_work.solo;
         std::vector<SWork> small;
-        for (int64_t i = 0; i < ns; i += SB_WAVES) small.push_back(SWork{-1, int32_t(nt + np + i)});
-        for (int64_t i = 0; i < np; i += SB_WAVES / 2) small.push_back(SWork{-2, int32_t(nt + i)});
+        auto add = [&](int64_t first, int64_t n, int32_t waves) {  // sorted by k-steps
+            int64_t i = first;
+            for (; i < first + n && B.blocks[size_t(B.work[size_t(i)].blk)].nk >= SB_SHARE; ++i)
+                small.push_back(SWork{-2 - waves, int32_t(i)});
+            for (; i < first + n; i += SB_WAVES / waves) small.push_back(SWork{-waves, int32_t(i)});
+        };
+        add(nt + np, ns, 1);
+        add(nt, np, 2);
         B.launch.reserve(size_t(nt) + small.size());
         size_t q = 0;
         for (int64_t i0 = 0; i0 < nt; i0 += 32) {
@@ -1753,12 +1765,13 @@ void check_sblocks(SBlockTable const& B, uint64_t t_size, uint64_t s_size) {
                     bad = std::max(bad, 4);
                 continue;
             }
-            const int64_t lo = l.blk == -1 ? nt + np : nt, hi = l.blk == -1 ? n : nt + np;
-            if (l.blk < -2 || l.n0 < lo || l.n0 >= hi) {
+            const int64_t waves = l.blk < -2 ? -int64_t(l.blk) - 2 : -l.blk, per = l.blk < -2 ? 1 : SB_WAVES / waves;
+            const int64_t lo = waves == 1 ? nt + np : nt, hi = waves == 1 ? n : nt + np;
+            if (waves > 2 || l.n0 < lo || l.n0 >= hi) {
                 bad = std::max(bad, 4);
                 continue;
             }
-            for (int64_t i = l.n0; i < std::min<int64_t>(hi, l.n0 + (l.blk == -1 ? SB_WAVES : SB_WAVES / 2)); ++i, ++items) {
+            for (int64_t i = l.n0; i < std::min<int64_t>(hi, l.n0 + per); ++i, ++items) {
                 if (small[size_t(i - nt)]) bad = std::max(bad, 4);
                 small[size_t(i - nt)] = 1;
             }
@@ -1783,7 +1796,8 @@ void check_sblocks(SBlockTable const& B, uint64_t t_size, uint64_t s_size) {
         }
     }
     for (SSmallWork const& w : B.small_work) {
-        bool ok = w.lg >= 0 && (1 << w.lg) <= SMALL_LINE_LANES && w.n > 0 && w.n <= (SMALL_LINE_LANES >> w.lg) &&
+        bool ok = w.lg >= 0 && w.ts >= 0 && w.lg + w.ts <= 30 && (1 << (w.lg + w.ts)) <= SMALL_LINE_LANES && w.n > 0 &&
+                  w.n <= (SMALL_LINE_LANES >> (w.lg + w.ts)) &&
                   w.line0 >= 0 && int64_t(w.line0) + w.n <= nsl;
         for (int32_t q = 0; ok && q < w.n; ++q) {
             SLine const& l = B.small_lines[size_t(w.line0 + q)];

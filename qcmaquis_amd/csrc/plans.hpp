@@ -130,18 +130,25 @@ struct SWork {
 // Work items by the waves that share one: tiles of more than 64 elements on the four waves of a
 // workgroup, of 33 to 64 on two, of at most 32 on one; the work list holds them in this order.  The
 // launch list has one entry per workgroup: a team's work item itself, or for workgroups of smaller
-// items (blk < 0) the first of its items (work[n0]) with -blk = 1 (one wave each) or 2.
+// items (blk < 0) the first of its items (work[n0]) with -blk = 1 (one wave each) or 2, or 3 or 4
+// where it runs this item alone, of one wave or of two, its k-steps shared out (SB_SHARE).
 struct SWorkCounts {
     int32_t team = 0, pair = 0, solo = 0;
 };
 constexpr int SB_WAVES = 4;  // waves of a term-sum workgroup
+// An item of one or two waves with at least this many k-steps has a workgroup to itself, its k-steps in
+// equal shares for four waves or two pairs (launch entry -2 - waves): the longest lists, several
+// hundred k-steps, are otherwise the last to end.  18 orbitals and M = 128, all tiles in blocks, term
+// sum in us from 9999 / 64 / 32 / 16 k-steps: 299 / 252 / 255 / 303; 12 and M = 96 91 / 65 / 67 / 71;
+// 18 and M = 509, where other work hides the long lists, 819 / 818 / 834 / 857
+constexpr int SB_SHARE = 64;
 // Lines marked SLINE_SMALL (tiles of at most SMALL_LINE_LANES elements) are summed term by term:
-// each line gets a power-of-two group of lanes (one lane per tile element) and a workgroup of 256
-// lanes takes 256 / group consecutive lines of one group size (lines sorted by group size, then by
-// term count, so the lanes of a wave run loops of similar length).
+// each line gets a power-of-two group of lanes, one lane per tile element, and as many such groups,
+// each with a share of the terms, as leave a lane SMALL_LINE_DEPTH terms (up to a workgroup's lanes).
+// A work item is the consecutive lines of one kind that a workgroup of 256 lanes holds.
 struct SSmallWork {
     int32_t line0, n;         // first line (small line table) and number of lines
-    int32_t lg, pad;          // log2 of the lanes per line
+    int32_t lg, ts;           // log2 of the lanes per tile (one an element) and of the shares of its terms
 };
 struct SBlockTable {
     std::vector<SBlock> blocks;
@@ -176,6 +183,7 @@ std::vector<GemmDesc> adjoint_y_gemms(std::vector<GemmDesc> const& c_gemms);
 std::vector<TermGradWork> term_grad_work(HostTable<SLine> const& lines, size_t l0, size_t l1);
 // lanes of a workgroup of the small-tile term sum; tiles up to this many elements can go there
 constexpr int SMALL_LINE_LANES = 256;
+constexpr int SMALL_LINE_DEPTH = 4;  // terms a lane sums before a line gets twice the lanes
 // work items cover SBLOCK_ELEMS consecutive tile elements of one block
 constexpr int SBLOCK_ELEMS = 128;
 // the block term sum loads one element past a tile of odd size: T buffers are that much longer
@@ -258,9 +266,12 @@ uint64_t gemm_stage_key(std::vector<GemmDesc> const& probs);
 // consecutive blocks of one tile shape (0: block by block)
 SBlockTable build_sblocks(HostTable<SLine> const& lines, HostTable<STerm> const& terms, int32_t panel = 0);
 // small-tile limit of the lines [l0, l1) of one site problem under the automatic rule: 64 when
-// their mean tile has at most 16 elements (then the 16-line blocks mostly hold tiles a few
-// elements wide, whose dense coefficient blocks cost more than the terms), else 0
-int32_t auto_small_tile_max(HostTable<SLine> const& lines, size_t l0, size_t l1);
+// their mean tile has at most 16 elements and the plan at most SMALL_TERMS_MAX terms (n_terms; 0:
+// those of the lines count), else 0.  Then the blocks are too few to fill the device: 8 orbitals and
+// M = 40 (0.2 million terms) take 10.5 us term by term, 30 in blocks; 12 and M = 96 (2.0 million)
+// 103 and 65, 18 and M = 128 (21 million) 496 and 252, as a block reads a tile once for 64 lines
+constexpr uint64_t SMALL_TERMS_MAX = 1u << 19;
+int32_t auto_small_tile_max(HostTable<SLine> const& lines, size_t l0, size_t l1, uint64_t n_terms = 0);
 // marks the lines [l0, l1) whose tiles have 1 .. limit elements SLINE_SMALL (limit <= 256)
 void mark_small_lines(HostTable<SLine>& lines, size_t l0, size_t l1, int32_t limit);
 void check_sblocks(SBlockTable const& B, uint64_t t_size, uint64_t s_size);

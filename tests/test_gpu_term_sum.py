@@ -2,7 +2,8 @@
 s x s elements with s*s around 32 (one wave), 64 (two waves) and 128 (a workgroup's range), single
 elements, odd sizes (an element pair past the tile's end) and coefficient tables longer than one
 staging pass.  FP64 to 1e-12 of the largest element (sums of a few thousand products, 2^-53 each),
-FP32 to 1e-5 (the mixed-precision bound of the other parity tests)."""
+FP32 to 1e-5 (the mixed-precision bound of the other parity tests).  The same term by term, at the edges
+of its lane groups and of the shares of a line's terms (lines of 1 to several hundred terms)."""
 import numpy as np
 import pytest
 
@@ -14,8 +15,7 @@ from tests.chains import oracle_left, oracle_right, rel_err
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("s,D", [(s, 24) for s in (1, 2, 5, 6, 8, 9, 11, 12, 17)] + [(1, 64), (12, 64)])
-def test_block_sum_tile_sizes(oracle_lib, ctx2u1, s, D):
+def run(oracle_lib, ctx, s, D, small_max):
     ch = Chain(np.random.default_rng(100 + s), abi.MQ_SYM_TWOU1, 4, (4, 4), s, D,
                phys=fuse_index(TWOU1_SITE, TWOU1_SITE), density=0.5, min_m=s)
     k = 2
@@ -24,17 +24,30 @@ def test_block_sum_tile_sizes(oracle_lib, ctx2u1, s, D):
     lay = ch.layouts[k]
     psi = np.random.default_rng(s).normal(size=lay.n)
     ref = oracle_lib.hpsi(ch.sym, ch.mpos[k], L, R, lay, psi)
-    ctx2u1.set_option(abi.MQ_OPT_SMALL_TILE_MAX, 0)  # every tile in blocks
+    ctx.set_option(abi.MQ_OPT_SMALL_TILE_MAX, small_max)
     try:
-        plan = HpsiPlan(ctx2u1, DeviceMPO(ctx2u1, ch.mpos[k]), DeviceBoundary.upload(ctx2u1, L),
-                        DeviceBoundary.upload(ctx2u1, R), lay)
+        plan = HpsiPlan(ctx, DeviceMPO(ctx, ch.mpos[k]), DeviceBoundary.upload(ctx, L), DeviceBoundary.upload(ctx, R), lay)
     finally:
-        ctx2u1.set_option(abi.MQ_OPT_SMALL_TILE_MAX, abi.MQ_SMALL_TILE_AUTO)
+        ctx.set_option(abi.MQ_OPT_SMALL_TILE_MAX, abi.MQ_SMALL_TILE_AUTO)
     st = plan.stats()
     err = rel_err(plan.apply(psi), ref)
     err32 = rel_err(plan.apply(psi, abi.MQ_PREC_FP32), ref)
-    print(f"tiles {s}x{s}: {st['n_sblocks']} blocks, max union {st['max_union_tiles']}, FP64 {err:.1e}, FP32 {err32:.1e}",
-          flush=True)
+    print(f"tiles {s}x{s}: {st['n_sblocks']} blocks, {st['small_lines']} small lines, max union {st['max_union_tiles']}, "
+          f"FP64 {err:.1e}, FP32 {err32:.1e}", flush=True)
+    return st, err, err32
+
+
+@pytest.mark.parametrize("s,D", [(s, 24) for s in (1, 2, 5, 6, 8, 9, 11, 12, 17)] + [(s, 64) for s in (1, 5, 6, 8, 12)])
+def test_block_sum_tile_sizes(oracle_lib, ctx2u1, s, D):
+    st, err, err32 = run(oracle_lib, ctx2u1, s, D, 0)  # every tile in blocks
     assert st["small_lines"] == 0 and st["n_sblocks"] > 0
-    assert D < 64 or st["max_union_tiles"] > 4 * 64  # more k-steps than one staging pass holds
+    # 64 k-steps of four tiles: shared out in tiles of up to 64 elements, more than one staging pass in larger ones
+    assert D < 64 or st["max_union_tiles"] >= 4 * 64 + (s > 8)
+    assert err < 1e-12 and err32 < 1e-5
+
+
+@pytest.mark.parametrize("s,D", [(1, 24), (1, 64), (2, 64), (3, 24), (5, 24), (8, 64), (9, 24), (11, 64), (16, 64)])
+def test_small_line_groups(oracle_lib, ctx2u1, s, D):
+    st, err, err32 = run(oracle_lib, ctx2u1, s, D, 256)  # every tile term by term
+    assert st["n_sblocks"] == 0 and st["small_lines"] > 0
     assert err < 1e-12 and err32 < 1e-5
