@@ -16,6 +16,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <tuple>
 #include <unordered_map>
 #include <vector>
 
@@ -28,12 +29,16 @@
 
 using namespace mq;
 
+// dot product partials of a context: one launch of products
+constexpr int DWORK_PARTIALS = VEC_MAX * DOT_BLOCKS;
+
 struct mq_ctx_s {
     int device = 0;
     Sym sym = Sym::TwoU1;
     hipStream_t stream = nullptr;
     std::string err;
-    double* dwork = nullptr;  // DOT_BLOCKS partials + 64 scalars
+    double* dwork = nullptr;  // DWORK_PARTIALS partials + 64 scalars
+    double* hscal = nullptr;  // VEC_MAX scalars in pinned host memory that kernels write
     bool plain_tables = false;         // MQ_OPT_PLAIN_TABLES
     int32_t small_tile_max = MQ_SMALL_TILE_AUTO;  // MQ_OPT_SMALL_TILE_MAX
     int32_t chunk_mb = MQ_CHUNK_AUTO;             // MQ_OPT_CHUNK_MB
@@ -482,6 +487,7 @@ struct mq_hpsi_plan_s {
     double* rown = nullptr;      // right boundaries copied into the plan (batch plans)
     std::vector<int64_t> inst_off;    // psi offset of each instance, and psi_n (batch plans)
     int64_t* d_inst_off = nullptr;    // the same on the device
+    double* batch_dots = nullptr;     // pinned host memory for VEC_MAX products of every instance, made on first use
     double build_seconds = 0, seconds_tables = 0, seconds_blocks = 0, seconds_plain = 0;
     uint64_t small_lines = 0, small_terms = 0, small_gathered = 0;
     // per-task tables of MQ_PREC_FP64_PLAIN (MQ_OPT_PLAIN_TABLES)
@@ -571,7 +577,9 @@ int mq_ctx_create(int device, int symmetry, mq_ctx_t* out) {
     c->sym = Sym(symmetry);
     int rc = guarded(c, [&] {
         hipcheck(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "stream create");
-        c->dwork = dev_alloc<double>(DOT_BLOCKS + 64);
+        c->dwork = dev_alloc<double>(DWORK_PARTIALS + 64);
+        hipcheck(hipHostMalloc(reinterpret_cast<void**>(&c->hscal), VEC_MAX * sizeof(double), hipHostMallocDefault),
+                 "pinned scalars");
         c->noalloc_scratch = noalloc_scratch_of(device);
     });
     if (rc != MQ_OK) {
@@ -587,6 +595,7 @@ int mq_ctx_destroy(mq_ctx_t ctx) {
     int rc = guarded(ctx, [&] {
         (void)hipStreamSynchronize(ctx->stream);
         dev_free(ctx->dwork);
+        if (ctx->hscal) (void)hipHostFree(ctx->hscal);
         {
             DevCache& c = devcache();
             std::lock_guard<std::mutex> lock(c.m);
@@ -1890,6 +1899,7 @@ int mq_hpsi_plan_destroy(mq_hpsi_plan_t p) {
         dev_free(p->plain.terms);
         dev_free(p->rown);
         dev_free(p->d_inst_off);
+        if (p->batch_dots) (void)hipHostFree(p->batch_dots);
     });
     delete p;
     return rc;
@@ -1975,7 +1985,8 @@ static void davidson_core(mq_hpsi_plan_t p, const double* psi0, int n_ortho, con
             bufs.push_back(dev_alloc<double>(n));
             return bufs.back();
         };
-        double* sc = p->ctx->dwork + DOT_BLOCKS;  // device scalars
+        double* sc = p->ctx->dwork + DWORK_PARTIALS;  // device scalars
+        double* hsc = p->ctx->hscal;
         double* work = p->ctx->dwork;
         double hpsi_s = 0;
         // GMRES steps of the correction equation (ietl_jcd_gmres; 0 = the plain correction)
@@ -1996,26 +2007,24 @@ static void davidson_core(mq_hpsi_plan_t p, const double* psi0, int n_ortho, con
                 hipcheck(hipMemcpyAsync(O[k], ortho[k], n * sizeof(double), hipMemcpyHostToDevice, s), "upload");
             }
             hipcheck(hipMemcpyAsync(V[0], psi0, n * sizeof(double), hipMemcpyHostToDevice, s), "upload");
+            // out[i] = x(i) . y(i) for i < count: up to VEC_MAX products in one launch pair, one wait
+            auto dots_host = [&](int count, auto x_of, auto y_of, double* out) {
+                for (int c0 = 0; c0 < count; c0 += VEC_MAX) {
+                    const int cn = std::min(VEC_MAX, count - c0);
+                    VecPairs v{};
+                    for (int i = 0; i < cn; ++i) {
+                        v.x[i] = x_of(c0 + i);
+                        v.y[i] = y_of(c0 + i);
+                    }
+                    hipcheck(launch_dots(v, cn, n, work, hsc, s), "dot");
+                    hipcheck(hipStreamSynchronize(s), "dot");
+                    std::copy(hsc, hsc + cn, out + c0);
+                }
+            };
             auto dot_host = [&](const double* x, const double* y) {
                 double h;
-                hipcheck(launch_dot(x, y, n, work, sc, s), "dot");
-                hipcheck(hipMemcpyAsync(&h, sc, sizeof(double), hipMemcpyDeviceToHost, s), "dot");
-                hipcheck(hipStreamSynchronize(s), "dot");
+                dots_host(1, [&](int) { return x; }, [&](int) { return y; }, &h);
                 return h;
-            };
-            // out[i] = x(i) . y(i) for i < count: the products into device scalars (one batch of at
-            // most DOT_BATCH at a time), then one download and one wait per batch
-            constexpr int SC_BATCH = 8, DOT_BATCH = 48;
-            static_assert(SC_BATCH + DOT_BATCH <= 64, "device scalars of the context");
-            auto dots_host = [&](int count, auto x_of, auto y_of, double* out) {
-                for (int c0 = 0; c0 < count; c0 += DOT_BATCH) {
-                    const int cn = std::min(DOT_BATCH, count - c0);
-                    for (int i = 0; i < cn; ++i)
-                        hipcheck(launch_dot(x_of(c0 + i), y_of(c0 + i), n, work, sc + SC_BATCH + i, s), "dot");
-                    hipcheck(hipMemcpyAsync(out + c0, sc + SC_BATCH, cn * sizeof(double), hipMemcpyDeviceToHost, s),
-                             "dot");
-                    hipcheck(hipStreamSynchronize(s), "dot");
-                }
             };
             // y -= (x.y)/(x.x) x   with coefficients kept on the device
             auto subtract_along = [&](double* y, const double* x, bool normalized) {
@@ -2106,13 +2115,26 @@ static void davidson_core(mq_hpsi_plan_t p, const double* psi0, int n_ortho, con
             while (true) {
                 double* t = V[it];
                 // modified Gram-Schmidt with one refinement when the norm collapses (jacobi.h:409-415)
-                double tau = std::sqrt(dot_host(t, t));
-                for (int i = 0; i < it; ++i) subtract_along(t, V[i], true);
-                if (std::sqrt(dot_host(t, t)) < 0.25 * tau)
-                    for (int i = 0; i < it; ++i) subtract_along(t, V[i], true);
+                double tt = 0;  // t . t, or < 0 when t has changed since
+                if (it == 0) {
+                    tt = dot_host(t, t);
+                } else {
+                    hipcheck(launch_gram_schmidt(t, V.data(), it, n, work, hsc, s), "gram-schmidt");
+                    hipcheck(hipStreamSynchronize(s), "gram-schmidt");
+                    tt = hsc[1];
+                    if (std::sqrt(tt) < 0.25 * std::sqrt(hsc[0])) {
+                        for (int i = 0; i < it; ++i) subtract_along(t, V[i], true);
+                        tt = -1;
+                    }
+                }
                 project(t);
-                hipcheck(launch_dot(t, t, n, work, sc, s), "dot");
-                hipcheck(launch_scale_rsqrt(t, n, sc, s), "scale");
+                if (no == 0 && tt >= 0) {
+                    const double inv = 1.0 / std::sqrt(tt);
+                    hipcheck(launch_lincomb(t, &t, &inv, 1, n, s), "scale");
+                } else {
+                    hipcheck(launch_dot(t, t, n, work, sc, s), "dot");
+                    hipcheck(launch_scale_rsqrt(t, n, sc, s), "scale");
+                }
                 auto h0 = std::chrono::steady_clock::now();
                 hpsi_run(p, t, VA[it], prec);
                 hipcheck(hipStreamSynchronize(s), "hpsi");
@@ -2129,25 +2151,29 @@ static void davidson_core(mq_hpsi_plan_t p, const double* psi0, int n_ortho, con
                         Ms[size_t(i) * dim + j] = Ms[size_t(j) * dim + i] = M[size_t(i) * max_iter + j];
                 small_sym_lowest(Ms, dim, theta, svec);
                 // u = V s, uA = VA s
-                hipcheck(launch_axpby(u, V[0], n, 0.0, svec[0], s), "axpby");
-                hipcheck(launch_axpby(r, VA[0], n, 0.0, svec[0], s), "axpby");
-                for (int j = 1; j < dim; ++j) {
-                    hipcheck(launch_axpby(u, V[j], n, 1.0, svec[j], s), "axpby");
-                    hipcheck(launch_axpby(r, VA[j], n, 1.0, svec[j], s), "axpby");
+                hipcheck(launch_lincomb(u, V.data(), svec.data(), dim, n, s), "ritz vector");
+                std::vector<double*> ops(VA.begin(), VA.begin() + dim);
+                std::vector<double> cf(svec);
+                if (no == 0) {  // r = uA - theta u
+                    ops.push_back(u);
+                    cf.push_back(-theta);
                 }
-                project(r);
-                hipcheck(launch_axpby(r, u, n, 1.0, -theta, s), "axpby");  // r = uA - theta u
+                hipcheck(launch_lincomb(r, ops.data(), cf.data(), int(ops.size()), n, s), "residual");
+                if (no > 0) {
+                    project(r);
+                    hipcheck(launch_axpby(r, u, n, 1.0, -theta, s), "axpby");
+                }
                 ++it;
-                rnorm = std::sqrt(dot_host(r, r));
+                double du[3];  // r.r, r.u, u.u
+                dots_host(3, [&](int i) { return i < 2 ? (const double*)r : (const double*)u; },
+                          [&](int i) { return i < 1 ? (const double*)r : (const double*)u; }, du);
+                rnorm = std::sqrt(du[0]);
                 bool conv = rnorm <= tol_run * std::fabs(theta) || rnorm < tol_run;  // iteration.h:57
                 if (conv || it >= iters) break;
                 // correction t = -r + (r.u)/(u.u) u  (jcd_gmres_solver with no GMRES steps, jacobi.h:152-156)
-                double du[2];
-                dots_host(2, [&](int i) { return i == 0 ? (const double*)r : (const double*)u; },
-                          [&](int) { return (const double*)u; }, du);
-                const double dru = du[0], duu = du[1];
-                hipcheck(launch_axpby(V[it], r, n, 0.0, -1.0, s), "axpby");
-                hipcheck(launch_axpby(V[it], u, n, 1.0, dru / duu, s), "axpby");
+                const double* ru[2] = {r, u};
+                const double co[2] = {-1.0, du[1] / du[2]};
+                hipcheck(launch_lincomb(V[it], ru, co, 2, n, s), "correction");
                 // with GMRES steps, that is the start of an approximate solution of the correction
                 // equation to the tolerance 2^-(it+1) (jcd_gmres_solver, jacobi.h:126-164)
                 if (gm > 0) gmres(V[it], prec, theta, 1.0 / std::pow(2.0, double(it + 1)));
@@ -2247,31 +2273,30 @@ extern "C" int mq_davidson_batch(mq_hpsi_plan_t p, const double* psi0, double to
             for (int i = 0; i < max_iter; ++i) { V[i] = alloc(n); VA[i] = alloc(n); }
             double* u = alloc(n);
             double* r = alloc(n);
-            double* part = alloc(uint64_t(ns) * SEG_CHUNKS);
-            // dot results: up to max_iter + 1 rows of ns; coefficient arrays a, b
-            double* dres = alloc(uint64_t(max_iter + 1) * ns);
-            double* ca = alloc(uint64_t(ns));
-            double* cb = alloc(uint64_t(ns));
-            std::vector<double> hres(size_t(max_iter + 1) * ns);
+            double* part = alloc(uint64_t(VEC_MAX) * ns * SEG_CHUNKS);
+            if (!p->batch_dots)
+                hipcheck(hipHostMalloc(reinterpret_cast<void**>(&p->batch_dots), size_t(VEC_MAX) * ns * sizeof(double),
+                                       hipHostMallocDefault), "pinned products");
+            const double* hres = p->batch_dots;
             hipcheck(hipMemcpyAsync(V[0], psi0, n * sizeof(double), hipMemcpyHostToDevice, s), "upload");
             hipcheck(hipStreamSynchronize(s), "upload");
-            // k dots (x_j . y_j, j < k) of every instance, one download
+            // k dots (x_j . y_j, j < k) of every instance, VEC_MAX at a time
             auto dots = [&](std::vector<std::pair<const double*, const double*>> const& xy) {
-                for (size_t j = 0; j < xy.size(); ++j)
-                    hipcheck(launch_seg_dot(xy[j].first, xy[j].second, off, ns, part, dres + j * ns, s), "dot");
-                hipcheck(hipMemcpyAsync(hres.data(), dres, xy.size() * ns * sizeof(double), hipMemcpyDeviceToHost, s),
-                         "dot");
-                hipcheck(hipStreamSynchronize(s), "dot");
                 std::vector<std::vector<double>> outv(xy.size());
-                for (size_t j = 0; j < xy.size(); ++j) outv[j].assign(hres.begin() + j * ns, hres.begin() + (j + 1) * ns);
+                for (size_t j0 = 0; j0 < xy.size(); j0 += VEC_MAX) {
+                    const int m = int(std::min<size_t>(VEC_MAX, xy.size() - j0));
+                    VecPairs v{};
+                    for (int j = 0; j < m; ++j) std::tie(v.x[j], v.y[j]) = xy[j0 + size_t(j)];
+                    hipcheck(launch_seg_dots(v, m, off, ns, part, p->batch_dots, s), "dot");
+                    hipcheck(hipStreamSynchronize(s), "dot");
+                    for (int j = 0; j < m; ++j)
+                        outv[j0 + size_t(j)].assign(hres + size_t(j) * ns, hres + size_t(j + 1) * ns);
+                }
                 return outv;
             };
-            // y_i = a_i y_i + b_i x_i (the coefficient uploads complete before the host vectors go)
+            // y_i = a_i y_i + b_i x_i
             auto axpby = [&](double* y, const double* x, std::vector<double> const& a, std::vector<double> const& b) {
-                hipcheck(hipMemcpyAsync(ca, a.data(), ns * sizeof(double), hipMemcpyHostToDevice, s), "coef");
-                hipcheck(hipMemcpyAsync(cb, b.data(), ns * sizeof(double), hipMemcpyHostToDevice, s), "coef");
-                hipcheck(launch_seg_axpby(y, x, off, ns, ca, cb, s), "axpby");
-                hipcheck(hipStreamSynchronize(s), "axpby");
+                hipcheck(launch_seg_axpby(y, x, off, ns, a.data(), b.data(), s), "axpby");
             };
             std::vector<double> theta(ns, 0.0), rnorm(ns, 0.0);
             std::vector<int32_t> its(ns, 0);
@@ -2303,8 +2328,10 @@ extern "C" int mq_davidson_batch(mq_hpsi_plan_t p, const double* psi0, double to
                         again[i] = active[i] && std::sqrt(nn[i]) < 0.25 * std::sqrt(tau[i]);
                         any |= again[i] != 0;
                     }
-                    if (any) gs_pass(again);
-                    nn = dots({{t, t}})[0];
+                    if (any) {
+                        gs_pass(again);
+                        nn = dots({{t, t}})[0];
+                    }
                     for (int i = 0; i < ns; ++i) {
                         am[i] = 0.0;
                         bm[i] = active[i] ? 1.0 / std::sqrt(nn[i]) : 0.0;  // inactive: t = 0, so H t = 0
@@ -2340,7 +2367,8 @@ extern "C" int mq_davidson_batch(mq_hpsi_plan_t p, const double* psi0, double to
                     for (int i = 0; i < ns; ++i) bm[i] = active[i] ? -theta[i] : 0.0;
                     axpby(r, u, one, bm);  // r = uA - theta u
                     ++it;
-                    auto rr = dots({{r, r}})[0];
+                    auto ru = dots({{r, u}, {u, u}, {r, r}});
+                    auto const& rr = ru[2];
                     bool any_active = false;
                     for (int i = 0; i < ns; ++i) {
                         if (!active[i]) continue;
@@ -2351,7 +2379,6 @@ extern "C" int mq_davidson_batch(mq_hpsi_plan_t p, const double* psi0, double to
                     }
                     if (!any_active || it >= iters) break;
                     // correction t = -r + (r.u)/(u.u) u of the active instances
-                    auto ru = dots({{r, u}, {u, u}});
                     for (int i = 0; i < ns; ++i) {
                         am[i] = 0.0;
                         bm[i] = active[i] ? -1.0 : 0.0;

@@ -642,6 +642,7 @@ __device__ inline double block_sum(double v) {
     __shared__ double red[DOT_THREADS / 64];
     for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
     int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    __syncthreads();  // an earlier sum has been read
     if (lane == 0) red[w] = v;
     __syncthreads();
     double r = 0.0;
@@ -650,22 +651,74 @@ __device__ inline double block_sum(double v) {
     return r;
 }
 
-__global__ __launch_bounds__(DOT_THREADS) void dot_partial_kernel(const double* __restrict__ x,
-                                                                  const double* __restrict__ y, uint64_t n,
-                                                                  double* __restrict__ work) {
+__device__ inline double dot_share(const double* __restrict__ x, const double* __restrict__ y, uint64_t n) {
     double s = 0.0;
     for (uint64_t i = uint64_t(blockIdx.x) * DOT_THREADS + threadIdx.x; i < n; i += uint64_t(gridDim.x) * DOT_THREADS)
         s += x[i] * y[i];
-    double r = block_sum(s);
+    return block_sum(s);
+}
+
+// the sum of a product's partials (thread 0)
+__device__ inline double dot_total(const double* __restrict__ work) {
+    double s = 0.0;
+    for (int i = threadIdx.x; i < DOT_BLOCKS; i += DOT_THREADS) s += work[i];
+    return block_sum(s);
+}
+
+__global__ __launch_bounds__(DOT_THREADS) void dot_partial_kernel(const double* __restrict__ x,
+                                                                  const double* __restrict__ y, uint64_t n,
+                                                                  double* __restrict__ work) {
+    const double r = dot_share(x, y, n);
     if (threadIdx.x == 0) work[blockIdx.x] = r;
 }
 
-__global__ __launch_bounds__(DOT_THREADS) void dot_final_kernel(const double* __restrict__ work, int nparts,
-                                                                double* __restrict__ out) {
+// The solvers' vectors are short (1e4 to 1e6 elements), so their kernels cost their launches: one by one,
+// some 340 of 2 to 3 us, and the gaps between them, in eight Jacobi-Davidson iterations of 14 orbitals
+// and M = 256.  Products that do not depend on each other share a launch (blockIdx.y: which), a
+// Gram-Schmidt step is one kernel, linear combinations are formed in one pass, and results for the host
+// go to pinned memory without a copy: the call takes 3.5 ms instead of 4.9 (H*psi 2.7 of them).
+__global__ __launch_bounds__(DOT_THREADS) void dots_partial_kernel(VecPairs v, uint64_t n, double* __restrict__ work) {
+    const double r = dot_share(v.x[blockIdx.y], v.y[blockIdx.y], n);
+    if (threadIdx.x == 0) work[blockIdx.y * DOT_BLOCKS + blockIdx.x] = r;
+}
+
+// out[b] = the sum of the partials from work[b * stride]
+__global__ __launch_bounds__(DOT_THREADS) void dots_final_kernel(const double* __restrict__ work, int stride,
+                                                                 double* __restrict__ out) {
+    const double r = dot_total(work + int64_t(blockIdx.x) * stride);
+    if (threadIdx.x == 0) out[blockIdx.x] = r;
+}
+
+// t -= (v . t) v with the product's partials in `have`, then the partials of next . t into `want` (next
+// may be t); every workgroup adds the partials up for itself
+__global__ __launch_bounds__(DOT_THREADS) void gram_schmidt_kernel(double* t, const double* __restrict__ v, const double* next,
+                                                                   uint64_t n, const double* __restrict__ have,
+                                                                   double* __restrict__ want) {
+    __shared__ double coef;
+    const double total = dot_total(have);
+    if (threadIdx.x == 0) coef = -total;
+    __syncthreads();
+    const double c = coef;
     double s = 0.0;
-    for (int i = threadIdx.x; i < nparts; i += DOT_THREADS) s += work[i];
-    double r = block_sum(s);
-    if (threadIdx.x == 0) out[0] = r;
+    for (uint64_t i = uint64_t(blockIdx.x) * DOT_THREADS + threadIdx.x; i < n; i += uint64_t(gridDim.x) * DOT_THREADS) {
+        const double x = t[i] + c * v[i];
+        t[i] = x;
+        s += x * (next == t ? x : next[i]);
+    }
+    const double r = block_sum(s);
+    if (threadIdx.x == 0) want[blockIdx.x] = r;
+}
+
+struct VecList {
+    const double* p[VEC_MAX];
+    double c[VEC_MAX];
+};
+__global__ void lincomb_kernel(double* out, VecList v, int count, uint64_t n) {
+    for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += uint64_t(gridDim.x) * blockDim.x) {
+        double s = v.c[0] * v.p[0][i];
+        for (int j = 1; j < count; ++j) s += v.c[j] * v.p[j][i];
+        out[i] = s;
+    }
 }
 
 __global__ void axpy_dev_kernel(double* __restrict__ y, const double* __restrict__ x, uint64_t n,
@@ -676,35 +729,38 @@ __global__ void axpy_dev_kernel(double* __restrict__ y, const double* __restrict
 }
 
 // Segmented forms for a batch of independent vectors concatenated in one buffer (segment s is
-// elements off[s] .. off[s+1]-1; blockIdx.y = segment).  Dot: SEG_CHUNKS partial sums per
-// segment, then one thread per segment adds them in chunk order (deterministic).
-__global__ __launch_bounds__(DOT_THREADS) void seg_dot_partial_kernel(const double* __restrict__ x,
-                                                                      const double* __restrict__ y,
-                                                                      const int64_t* __restrict__ off,
-                                                                      double* __restrict__ part) {
+// elements off[s] .. off[s+1]-1; blockIdx.y = segment).  Dots (blockIdx.z = which): SEG_CHUNKS partial
+// sums per segment, then one thread per segment adds them in chunk order (deterministic).
+__global__ __launch_bounds__(DOT_THREADS) void seg_dots_partial_kernel(VecPairs v, const int64_t* __restrict__ off,
+                                                                       double* __restrict__ part) {
     const int seg = blockIdx.y;
     const int64_t a = off[seg], b = off[seg + 1];
+    const double *x = v.x[blockIdx.z], *y = v.y[blockIdx.z];
     double s = 0.0;
     for (int64_t i = a + int64_t(blockIdx.x) * DOT_THREADS + threadIdx.x; i < b; i += int64_t(SEG_CHUNKS) * DOT_THREADS)
         s += x[i] * y[i];
     double r = block_sum(s);
-    if (threadIdx.x == 0) part[int64_t(seg) * SEG_CHUNKS + blockIdx.x] = r;
+    if (threadIdx.x == 0) part[(int64_t(blockIdx.z) * gridDim.y + seg) * SEG_CHUNKS + blockIdx.x] = r;
 }
 
-__global__ void seg_dot_final_kernel(const double* __restrict__ part, int nseg, double* __restrict__ out) {
-    const int seg = int(blockIdx.x * blockDim.x + threadIdx.x);
-    if (seg >= nseg) return;
+__global__ void seg_dots_final_kernel(const double* __restrict__ part, int n, double* __restrict__ out) {
+    const int q = int(blockIdx.x * blockDim.x + threadIdx.x);
+    if (q >= n) return;
     double s = 0.0;
-    for (int c = 0; c < SEG_CHUNKS; ++c) s += part[int64_t(seg) * SEG_CHUNKS + c];
-    out[seg] = s;
+    for (int c = 0; c < SEG_CHUNKS; ++c) s += part[int64_t(q) * SEG_CHUNKS + c];
+    out[q] = s;
 }
 
+// the coefficients of SEG_COEFS consecutive segments travel with the launch
+constexpr int SEG_COEFS = 32;
+struct SegCoefs {
+    double a[SEG_COEFS], b[SEG_COEFS];
+};
 // segment s: y = a[s]*y + b[s]*x (y not read where a[s] == 0)
-__global__ void seg_axpby_kernel(double* __restrict__ y, const double* __restrict__ x, const int64_t* __restrict__ off,
-                                 const double* __restrict__ ca, const double* __restrict__ cb) {
+__global__ void seg_axpby_kernel(double* y, const double* x, const int64_t* __restrict__ off, SegCoefs k) {
     const int seg = blockIdx.y;
     const int64_t i0 = off[seg], i1 = off[seg + 1];
-    const double a = ca[seg], b = cb[seg];
+    const double a = k.a[seg], b = k.b[seg];
     for (int64_t i = i0 + int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < i1; i += int64_t(gridDim.x) * blockDim.x)
         y[i] = a == 0.0 ? b * x[i] : a * y[i] + b * x[i];
 }
@@ -844,7 +900,51 @@ hipError_t launch_reshape(const ReshapeSeg* segs, int32_t n_segs, const double* 
 
 hipError_t launch_dot(const double* x, const double* y, uint64_t n, double* work, double* out, hipStream_t stream) {
     hipLaunchKernelGGL(dot_partial_kernel, dim3(DOT_BLOCKS), dim3(DOT_THREADS), 0, stream, x, y, n, work);
-    hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(DOT_THREADS), 0, stream, work, DOT_BLOCKS, out);
+    hipLaunchKernelGGL(dots_final_kernel, dim3(1), dim3(DOT_THREADS), 0, stream, work, DOT_BLOCKS, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_dots(VecPairs const& v, int count, uint64_t n, double* work, double* out, hipStream_t stream) {
+    if (count <= 0) return hipSuccess;
+    if (count > VEC_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(dots_partial_kernel, dim3(DOT_BLOCKS, unsigned(count)), dim3(DOT_THREADS), 0, stream, v, n, work);
+    hipLaunchKernelGGL(dots_final_kernel, dim3(unsigned(count)), dim3(DOT_THREADS), 0, stream, work, DOT_BLOCKS, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_gram_schmidt(double* t, const double* const* v, int count, uint64_t n, double* work, double* out,
+                               hipStream_t stream) {
+    if (count <= 0) return hipErrorInvalidValue;
+    // partials: t . t before in part 0, the steps' products in 1 and 2 by turns, t . t after in 3
+    auto part = [&](int i) { return work + int64_t(i) * DOT_BLOCKS; };
+    VecPairs first{};
+    first.x[0] = first.y[0] = first.y[1] = t;
+    first.x[1] = v[0];
+    hipLaunchKernelGGL(dots_partial_kernel, dim3(DOT_BLOCKS, 2), dim3(DOT_THREADS), 0, stream, first, n, work);
+    for (int i = 0; i < count; ++i) {
+        const bool last = i + 1 == count;
+        hipLaunchKernelGGL(gram_schmidt_kernel, dim3(DOT_BLOCKS), dim3(DOT_THREADS), 0, stream, t, v[i],
+                           last ? t : v[i + 1], n, part(1 + i % 2), part(last ? 3 : 1 + (i + 1) % 2));
+    }
+    hipLaunchKernelGGL(dots_final_kernel, dim3(2), dim3(DOT_THREADS), 0, stream, work, 3 * DOT_BLOCKS, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_lincomb(double* out, const double* const* p, const double* c, int count, uint64_t n, hipStream_t stream) {
+    if (count <= 0) return hipErrorInvalidValue;
+    for (int j = 0; j < count;) {
+        VecList v{};
+        int m = 0;
+        if (j > 0) {  // the sum so far
+            v.p[m] = out;
+            v.c[m++] = 1.0;
+        }
+        for (; j < count && m < VEC_MAX; ++j, ++m) {
+            v.p[m] = p[j];
+            v.c[m] = c[j];
+        }
+        hipLaunchKernelGGL(lincomb_kernel, dim3(grid_for(n, 256)), dim3(256), 0, stream, out, v, m, n);
+    }
     return hipGetLastError();
 }
 
@@ -854,19 +954,28 @@ hipError_t launch_axpy_dev(double* y, const double* x, uint64_t n, const double*
     return hipGetLastError();
 }
 
-hipError_t launch_seg_dot(const double* x, const double* y, const int64_t* off, int nseg, double* part, double* out,
-                          hipStream_t stream) {
-    if (nseg <= 0) return hipSuccess;
-    hipLaunchKernelGGL(seg_dot_partial_kernel, dim3(SEG_CHUNKS, unsigned(nseg)), dim3(DOT_THREADS), 0, stream, x, y,
-                       off, part);
-    hipLaunchKernelGGL(seg_dot_final_kernel, dim3(unsigned((nseg + 255) / 256)), dim3(256), 0, stream, part, nseg, out);
+hipError_t launch_seg_dots(VecPairs const& v, int count, const int64_t* off, int nseg, double* part, double* out,
+                           hipStream_t stream) {
+    if (nseg <= 0 || count <= 0) return hipSuccess;
+    if (count > VEC_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(seg_dots_partial_kernel, dim3(SEG_CHUNKS, unsigned(nseg), unsigned(count)), dim3(DOT_THREADS), 0,
+                       stream, v, off, part);
+    hipLaunchKernelGGL(seg_dots_final_kernel, dim3(unsigned((count * nseg + 255) / 256)), dim3(256), 0, stream, part,
+                       count * nseg, out);
     return hipGetLastError();
 }
 
 hipError_t launch_seg_axpby(double* y, const double* x, const int64_t* off, int nseg, const double* a, const double* b,
                             hipStream_t stream) {
-    if (nseg <= 0) return hipSuccess;
-    hipLaunchKernelGGL(seg_axpby_kernel, dim3(SEG_CHUNKS, unsigned(nseg)), dim3(256), 0, stream, y, x, off, a, b);
+    for (int s0 = 0; s0 < nseg; s0 += SEG_COEFS) {
+        const int m = nseg - s0 < SEG_COEFS ? nseg - s0 : SEG_COEFS;
+        SegCoefs k{};
+        for (int i = 0; i < m; ++i) {
+            k.a[i] = a[s0 + i];
+            k.b[i] = b[s0 + i];
+        }
+        hipLaunchKernelGGL(seg_axpby_kernel, dim3(SEG_CHUNKS, unsigned(m)), dim3(256), 0, stream, y, x, off + s0, k);
+    }
     return hipGetLastError();
 }
 

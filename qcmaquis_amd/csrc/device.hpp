@@ -65,17 +65,33 @@ hipError_t launch_reshape(const ReshapeSeg* segs, int32_t n_segs, const double* 
 // out[0] = x . y  (deterministic two-level reduction; work holds DOT_BLOCKS partials)
 constexpr int DOT_BLOCKS = 512;
 hipError_t launch_dot(const double* x, const double* y, uint64_t n, double* work, double* out, hipStream_t stream);
+// several dots in a launch pair: out[j] = x[j] . y[j], j < count <= VEC_MAX (work holds count * DOT_BLOCKS
+// partials; out may be pinned host memory), each the same sum as launch_dot's
+constexpr int VEC_MAX = 16;
+struct VecPairs {
+    const double* x[VEC_MAX];
+    const double* y[VEC_MAX];
+};
+hipError_t launch_dots(VecPairs const& v, int count, uint64_t n, double* work, double* out, hipStream_t stream);
+// modified Gram-Schmidt of t against the unit vectors v[0 .. count), count > 0: t -= (v_i . t) v_i in turn, each
+// product of the t left by the one before; out[0], out[1] = t . t before and after (work holds 4 *
+// DOT_BLOCKS partials)
+hipError_t launch_gram_schmidt(double* t, const double* const* v, int count, uint64_t n, double* work, double* out,
+                               hipStream_t stream);
+// out = sum of c[j] p[j], j < count, in order (count >= 1); out may be one of the operands
+hipError_t launch_lincomb(double* out, const double* const* p, const double* c, int count, uint64_t n, hipStream_t stream);
 // y += coef * x with coef = sign * num[0] / (den ? den[0] : 1)  (coefficients stay on the device)
 hipError_t launch_axpy_dev(double* y, const double* x, uint64_t n, const double* num, const double* den, double sign,
                            hipStream_t stream);
 // y = a*y + b*x (host scalars); a == 0 assigns b*x without reading y
 hipError_t launch_axpby(double* y, const double* x, uint64_t n, double a, double b, hipStream_t stream);
-// segmented forms over nseg (<= 65535) vectors concatenated in one buffer, segment s being
-// elements off[s] .. off[s+1]-1 (off on the device): out[s] = x_s . y_s (part holds
-// nseg * SEG_CHUNKS partials), and y_s = a[s]*y_s + b[s]*x_s (a, b on the device)
+// segmented forms over nseg vectors concatenated in one buffer, segment s being elements
+// off[s] .. off[s+1]-1 (off on the device): out[j * nseg + s] = x[j]_s . y[j]_s for j < count <= VEC_MAX
+// (part holds count * nseg * SEG_CHUNKS partials; out may be pinned host memory; nseg <= 65535), and
+// y_s = a[s]*y_s + b[s]*x_s (a, b on the host, read before the call returns; y not read where a[s] == 0)
 constexpr int SEG_CHUNKS = 64;
-hipError_t launch_seg_dot(const double* x, const double* y, const int64_t* off, int nseg, double* part, double* out,
-                          hipStream_t stream);
+hipError_t launch_seg_dots(VecPairs const& v, int count, const int64_t* off, int nseg, double* part, double* out,
+                           hipStream_t stream);
 hipError_t launch_seg_axpby(double* y, const double* x, const int64_t* off, int nseg, const double* a, const double* b,
                             hipStream_t stream);
 // x *= 1/sqrt(nrm2[0])
