@@ -75,7 +75,7 @@ __device__ inline void split_bf16(float x, short& hi, short& lo) {
 // per tile shape: B is staged for 128 columns of up to 128 rows instead of 64, waves of an item
 // no longer wait for the one with the most row steps, and the items of all heights share one launch
 // and one tail.  T / L*S stages in us before -> now: 8 orbitals, M = 40 8 / 23 -> 8 / 20;
-// 18, M = 509 323 / 412 -> 307 / 400; 20 with spins, M = 700 997 / 958 -> 913 / 901, M = 2048
+// 18, M = 509 323 / 412 -> 307 / 377; 20 with spins, M = 700 997 / 958 -> 912 / 880, M = 2048
 // 14.8 / 18.9 -> 13.8 / 15.1 ms.
 constexpr int GEMM_TILE = 128, GEMM_KS = 16, GEMM_THREADS = 512;
 template <class TI>
@@ -269,7 +269,11 @@ __global__ __launch_bounds__(GEMM_THREADS, 4) void gemm_kernel(const GemmDesc* _
     else gemm_tile<TI, TO, BF3, false, false>(lds, tile, g, rows, bases, ws);
 }
 
-// C tile = sum of its split partials, added in split order; blockIdx.y selects 256 elements of the tile
+// C tile = sum of its split partials, added in split order; blockIdx.y selects 256 elements of the tile.
+// Bound: the latency of the partials' loads, so REDUCE_U of them are in flight ahead of their sums.  L*S
+// stages in us with 1 / 4 / 8 / 16: 14 orbitals, M = 256 96 / 85 / 85 / 87, 18 and M = 509 401 / 384 / 377 /
+// 379, 18 and M = 128 56 / 49 / 48 / 51
+constexpr int REDUCE_U = 8;
 template <class TW, class TO>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmDesc* __restrict__ probs,
                                                           const GemmReduce* __restrict__ jobs, Bases bases,
@@ -286,7 +290,16 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmDesc* __rest
         const int m = m0 + mm, n = n0 + nn;
         if (m < g.M && n < g.N) {
             TW sum = 0;
-            for (int s = 0; s < job.nsplit; ++s) sum += ws[job.ws + s * tile_elems + idx];
+            const TW* p = ws + job.ws + idx;
+            int s = 0;
+            for (; s + REDUCE_U <= job.nsplit; s += REDUCE_U) {
+                TW v[REDUCE_U];
+#pragma unroll
+                for (int u = 0; u < REDUCE_U; ++u) v[u] = p[(s + u) * tile_elems];
+#pragma unroll
+                for (int u = 0; u < REDUCE_U; ++u) sum += v[u];
+            }
+            for (; s < job.nsplit; ++s) sum += p[s * tile_elems];
             C[m + int64_t(n) * g.ldc] = TO(sum);
         }
     }

@@ -222,7 +222,7 @@ struct GemmSchedule {
 // The choices of a grouped GEMM schedule that the tile autotuner varies.  target_items: workgroups
 // a stage should provide before K is split; min_chunk: shortest K range of a split tile (a multiple
 // of the K step 16).  L*S stages in us at targets
-// of 2048 / 4096: 18 orbitals and M = 509 376 / 400, 20 with spins and M = 700 865 / 901, M = 2048
+// of 2048 / 4096: 18 orbitals and M = 509 376 / 400, 20 with spins and M = 700 865 / 901 (with a slower split sum), M = 2048
 // 15.5 / 15.1 ms (17.1 at 1024); the shorter ranges of 4096 keep the FP32 rounding down (18 orbitals,
 // M = 512: 4.3e-7 at 2048, 3.5e-7 at 4096)
 struct GemmPolicy {

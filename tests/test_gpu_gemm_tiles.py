@@ -14,9 +14,11 @@ from tests.chains import oracle_left, oracle_right, rel_err
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("s", [1, 3, 15, 16, 17, 31, 33, 64, 65, 97, 127, 128, 129, 140])
-def test_gemm_tile_edges(oracle_lib, ctx2u1, s):
-    ch = Chain(np.random.default_rng(200 + s), abi.MQ_SYM_TWOU1, 4, (2, 2), s, 6, min_m=s)
+# (12, 96), (17, 64) and (33, 48): reductions of a few thousand, split into more than eight ranges
+@pytest.mark.parametrize("s,D", [(s, 6) for s in (1, 3, 15, 16, 17, 31, 33, 64, 65, 97, 127, 128, 129, 140)] +
+                         [(12, 96), (17, 64), (33, 48)])
+def test_gemm_tile_edges(oracle_lib, ctx2u1, s, D):
+    ch = Chain(np.random.default_rng(200 + s), abi.MQ_SYM_TWOU1, 4, (2, 2), s, D, min_m=s)
     k = 2
     L = oracle_left(oracle_lib, ch, k + 1)
     R = oracle_right(oracle_lib, ch, k + 1)[k + 1]
