@@ -1929,24 +1929,33 @@ GemmSchedule build_gemm_schedule(std::vector<GemmDesc> const& probs, GemmPolicy 
                     S.ws_elems += uint64_t(splits) * bm * bn;
                 }
     }
-    // longest reductions first for load balance
-    for (auto& v : S.tiles)
-        std::stable_sort(v.begin(), v.end(), [](GemmTile const& a, GemmTile const& b) { return a.k1 - a.k0 > b.k1 - b.k0; });
     return S;
 }
 
 std::vector<GemmItem> gemm_items(std::vector<GemmDesc> const& probs, GemmSchedule const& sch) {
+    // runs of consecutive tiles of one amount of work (mostly a whole problem) are sorted, not the tiles
+    struct Run { int64_t work; int32_t sh; uint32_t first, n; };
+    std::vector<Run> runs;
+    for (int32_t sh = 0; sh < GEMM_N_SHAPES; ++sh) {
+        auto const& v = sch.tiles[sh];
+        require(v.size() < size_t(UINT32_MAX), "gemm schedule: more than 2^32 tiles");
+        for (size_t i = 0; i < v.size(); ++i) {
+            const int64_t work = int64_t(v[i].k1 - v[i].k0) * gemm_bm(sh);
+            if (i > 0 && runs.back().work == work) ++runs.back().n;
+            else runs.push_back(Run{work, sh, uint32_t(i), 1});
+        }
+    }
+    std::stable_sort(runs.begin(), runs.end(), [](Run const& a, Run const& b) { return a.work > b.work; });
     std::vector<GemmItem> out;
     out.reserve(size_t(sch.n_tiles()));
-    for (int sh = 0; sh < GEMM_N_SHAPES; ++sh) {
-        const int32_t bm = gemm_bm(sh), bn = gemm_bn(sh);
-        for (GemmTile const& t : sch.tiles[sh])
+    for (Run const& r : runs) {
+        const int32_t bm = gemm_bm(r.sh), bn = gemm_bn(r.sh);
+        for (uint32_t i = r.first; i < r.first + r.n; ++i) {
+            GemmTile const& t = sch.tiles[r.sh][i];
             out.push_back(GemmItem{t.prob, t.batch, t.tm * bm, std::min(bm, probs[size_t(t.prob)].M - t.tm * bm), t.tn * bn,
                                    t.k0, t.k1, bm, t.ws});
+        }
     }
-    std::stable_sort(out.begin(), out.end(), [](GemmItem const& a, GemmItem const& b) {
-        return int64_t(a.k1 - a.k0) * a.bm > int64_t(b.k1 - b.k0) * b.bm;
-    });
     return out;
 }
 
