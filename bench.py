@@ -1051,7 +1051,7 @@ def main():
                                   "formulation" % (s_bytes, st["t_elements"], st["s_line_elements"], st["n_sblocks"],
                                                    st["union_elements"], st["n_terms"], st["gathered_elements"])}
     # the dominant kernel: the term sum is one launch per H*psi and the largest single share of its
-    # time; the GEMM stages are spread over three tile-shape instances per stage and a reduce
+    # time; the GEMM stages are a launch per stage and a reduce
     dominant, other = rl_sasm, rl_gemm
     # HBM bytes per launch (per H*psi for the GEMM family) from the committed rocprofv3 counter runs
     # of this default workload (FETCH_SIZE / WRITE_SIZE scaled by a device-copy calibration)
