@@ -796,25 +796,28 @@ inline unsigned grid_for(uint64_t n, int threads, unsigned cap = 8192) {
     return unsigned(g > cap ? cap : g);
 }
 
-}  // namespace
-
-namespace {
+// launches a list of n workgroups of `threads` threads in pieces: run(first, count).  A launch takes
+// fewer than 2^32 threads along x, so the piece depends on the workgroup's size: 8.4 million of 512
+// threads, 16.8 million of 256.
+template <class F>
+void in_pieces(int64_t n, int threads, F&& run) {
+    const int64_t most = int64_t(0xffffffffu) / threads;
+    for (int64_t off = 0; off < n; off += most) run(off, unsigned(n - off < most ? n - off : most));
+}
 
 template <class TI, class TO, bool BF3 = false>
 void launch_gemm_t(const GemmDesc* probs, const GemmRow* rows, const GemmItem* items, int64_t n_items,
                    const GemmReduce* reduces, int64_t n_reduces, int32_t reduce_elems, void* ws, Bases bases,
                    hipStream_t stream) {
     TI* w = static_cast<TI*>(ws);
-    for (int64_t off = 0; off < n_items; off += 0x7fffffff) {
-        const int64_t cnt = n_items - off < 0x7fffffff ? n_items - off : 0x7fffffff;
-        hipLaunchKernelGGL((gemm_kernel<TI, TO, BF3>), dim3(unsigned(cnt)), dim3(GEMM_THREADS), 0, stream, probs, rows,
-                           items + off, bases, w);
-    }
-    for (int64_t off = 0; off < n_reduces; off += 0x7fffffff) {
-        const int64_t cnt = n_reduces - off < 0x7fffffff ? n_reduces - off : 0x7fffffff;
-        hipLaunchKernelGGL((gemm_reduce_kernel<TI, TO>), dim3(unsigned(cnt), unsigned((reduce_elems + 255) / 256)), dim3(256),
-                           0, stream, probs, reduces + off, bases, w);
-    }
+    in_pieces(n_items, GEMM_THREADS, [&](int64_t off, unsigned cnt) {
+        hipLaunchKernelGGL((gemm_kernel<TI, TO, BF3>), dim3(cnt), dim3(GEMM_THREADS), 0, stream, probs, rows, items + off,
+                           bases, w);
+    });
+    in_pieces(n_reduces, 256, [&](int64_t off, unsigned cnt) {
+        hipLaunchKernelGGL((gemm_reduce_kernel<TI, TO>), dim3(cnt, unsigned((reduce_elems + 255) / 256)), dim3(256), 0,
+                           stream, probs, reduces + off, bases, w);
+    });
 }
 
 }  // namespace
@@ -836,10 +839,9 @@ hipError_t launch_gemm(GemmPrec prec, const GemmDesc* probs, const GemmRow* rows
 
 hipError_t launch_slines(const SLine* lines, int64_t n_lines, const STerm* terms, const double* T, double* S,
                          hipStream_t stream) {
-    for (int64_t off = 0; off < n_lines; off += 0x7fffffff) {
-        int64_t cnt = n_lines - off < 0x7fffffff ? n_lines - off : 0x7fffffff;
-        hipLaunchKernelGGL(sline_kernel, dim3(unsigned(cnt)), dim3(256), 0, stream, lines + off, terms, T, S);
-    }
+    in_pieces(n_lines, 256, [&](int64_t off, unsigned cnt) {
+        hipLaunchKernelGGL(sline_kernel, dim3(cnt), dim3(256), 0, stream, lines + off, terms, T, S);
+    });
     return hipGetLastError();
 }
 
@@ -847,10 +849,10 @@ template <class T>
 hipError_t launch_sblocks(const SBlock* blocks, const SWork* launch, int64_t n_launch, const SWork* work, SWorkCounts n,
                           const int64_t* utile, const uint32_t* kstep, const T* ualpha, const int64_t* lsoff,
                           const int32_t* llds, const T* X, T* S, bool xcd_contiguous, hipStream_t stream) {
-    if (n_launch > 0x7fffffff) return hipErrorInvalidValue;
-    if (n_launch > 0)
-        hipLaunchKernelGGL(sblock_kernel<T>, dim3(unsigned(n_launch)), dim3(SB_THREADS), 0, stream, blocks, launch, work, n,
-                           utile, kstep, ualpha, lsoff, llds, X, S, int(xcd_contiguous));
+    in_pieces(n_launch, SB_THREADS, [&](int64_t off, unsigned cnt) {
+        hipLaunchKernelGGL(sblock_kernel<T>, dim3(cnt), dim3(SB_THREADS), 0, stream, blocks, launch + off, work, n, utile,
+                           kstep, ualpha, lsoff, llds, X, S, int(xcd_contiguous));
+    });
     return hipGetLastError();
 }
 template hipError_t launch_sblocks<double>(const SBlock*, const SWork*, int64_t, const SWork*, SWorkCounts,
@@ -863,11 +865,9 @@ template hipError_t launch_sblocks<float>(const SBlock*, const SWork*, int64_t, 
 template <class T>
 hipError_t launch_small_lines(const SSmallWork* work, int64_t n_work, const SLine* lines, const STerm* terms,
                               const T* X, T* S, hipStream_t stream) {
-    for (int64_t off = 0; off < n_work; off += 0x7fffffff) {
-        int64_t cnt = n_work - off < 0x7fffffff ? n_work - off : 0x7fffffff;
-        hipLaunchKernelGGL(small_lines_kernel<T>, dim3(unsigned(cnt)), dim3(SMALL_LINE_LANES), 0, stream, work + off,
-                           lines, terms, X, S);
-    }
+    in_pieces(n_work, SMALL_LINE_LANES, [&](int64_t off, unsigned cnt) {
+        hipLaunchKernelGGL(small_lines_kernel<T>, dim3(cnt), dim3(SMALL_LINE_LANES), 0, stream, work + off, lines, terms, X, S);
+    });
     return hipGetLastError();
 }
 template hipError_t launch_small_lines<double>(const SSmallWork*, int64_t, const SLine*, const STerm*, const double*,
@@ -878,11 +878,10 @@ template hipError_t launch_small_lines<float>(const SSmallWork*, int64_t, const 
 hipError_t launch_term_grad(const TermGradWork* work, int64_t n_work, const SLine* lines, const STerm* terms,
                             const uint32_t* src, const double* beta, const double* Y, const double* T, double* grad,
                             hipStream_t stream) {
-    for (int64_t off = 0; off < n_work; off += 0x7fffffff) {
-        const int64_t cnt = n_work - off < 0x7fffffff ? n_work - off : 0x7fffffff;
-        hipLaunchKernelGGL(term_grad_kernel, dim3(unsigned(cnt)), dim3(TERM_GRAD_THREADS), 0, stream, work + off, lines,
-                           terms, src, beta, Y, T, grad);
-    }
+    in_pieces(n_work, TERM_GRAD_THREADS, [&](int64_t off, unsigned cnt) {
+        hipLaunchKernelGGL(term_grad_kernel, dim3(cnt), dim3(TERM_GRAD_THREADS), 0, stream, work + off, lines, terms, src,
+                           beta, Y, T, grad);
+    });
     return hipGetLastError();
 }
 
