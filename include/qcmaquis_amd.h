@@ -82,10 +82,11 @@ extern "C" {
 #define MQ_OPT_SBLOCK_XCD 6    /* value 1: plans made afterwards give each XCD a contiguous range of
                                   the term sum's work items instead of every eighth (default 0) */
 #define MQ_OPT_AUTOTUNE 7      /* value 1: H*psi plans made afterwards choose the schedule of each
-                                  GEMM stage among the candidate tile rules by timing them, once per
-                                  key of the stage's (m, n, k) histogram; later stages with a known
-                                  key take the recorded pick without timing (mq_ctx_tuned lists
-                                  them).  Default 0: the default rule. */
+                                  GEMM stage among the candidate splits along K by timing those that
+                                  differ for it, once per key of the stage's (m, n, k) histogram;
+                                  later stages with a known key take the recorded pick without
+                                  timing (mq_ctx_tuned lists them).  T stages have no other split
+                                  than the default rule's.  Default 0: the default rule. */
 #define MQ_OPT_JCD_GMRES 8     /* value 0..64: GMRES steps of mq_davidson's correction equation (the
                                   reference's ietl_jcd_gmres; jcd_gmres_solver, ietl/jacobi.h:126-164,
                                   ietl_gmres, ietl/gmres.h:89-145); 0 (default): the plain correction

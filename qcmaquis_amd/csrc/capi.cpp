@@ -939,8 +939,9 @@ struct LpanelPart {
 };
 
 // GEMM tile autotuner: each GEMM stage of the plan whose histogram key the context has not seen
-// is timed under every schedule candidate (gemm_policy; one warm-up launch, then the faster of
-// two timed launches, HIP events on the context stream); the fastest is recorded for the key and
+// is timed under every schedule candidate that differs for it (gemm_candidates; one warm-up launch,
+// then the faster of two timed launches, HIP events on the context stream); the fastest is recorded
+// for the key and
 // a stage with a known key takes the recorded candidate.  The stage is re-uploaded with its
 // schedule unless that is the default one it already has.
 static void autotune_plan(mq_ctx_t ctx, mq_hpsi_plan_s* p, std::vector<std::vector<GemmDesc>> const& tgs,
@@ -986,10 +987,9 @@ static void autotune_plan(mq_ctx_t ctx, mq_hpsi_plan_s* p, std::vector<std::vect
                 auto it = ctx->tuned.find(key);
                 if (it == ctx->tuned.end()) {
                     mq_ctx_s::Tuned t{0, 1e30f, 0.0f};
-                    for (int cand = 0; cand < GEMM_N_POLICIES; ++cand) {
-                        GemmSchedule sch = build_gemm_schedule(descs, gemm_policy(cand));
+                    for (GemmCandidate const& cand : gemm_candidates(descs)) {
                         GemmStage tmp;
-                        tmp.upload(descs, rows, s, &sch);
+                        tmp.upload(descs, rows, s, &cand.schedule);
                         float ms = 0;
                         try {
                             ms = time_stage(tmp);
@@ -999,8 +999,8 @@ static void autotune_plan(mq_ctx_t ctx, mq_hpsi_plan_s* p, std::vector<std::vect
                             throw;
                         }
                         tmp.release();
-                        if (cand == 0) t.default_ms = ms;
-                        if (ms < t.best_ms) t.best_ms = ms, t.pick = cand;
+                        if (cand.policy == 0) t.default_ms = ms;
+                        if (ms < t.best_ms) t.best_ms = ms, t.pick = cand.policy;
                     }
                     it = ctx->tuned.emplace(key, t).first;
                 }

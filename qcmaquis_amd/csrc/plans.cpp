@@ -1845,6 +1845,29 @@ GemmPolicy gemm_policy(int i) {
     return p;
 }
 
+std::vector<GemmCandidate> gemm_candidates(std::vector<GemmDesc> const& probs) {
+    auto same_tile = [](GemmTile const& a, GemmTile const& b) {
+        return a.prob == b.prob && a.batch == b.batch && a.tm == b.tm && a.tn == b.tn && a.k0 == b.k0 && a.k1 == b.k1 &&
+               a.ws == b.ws;
+    };
+    // the split sums follow from the tiles
+    auto same = [&](GemmSchedule const& a, GemmSchedule const& b) {
+        for (int sh = 0; sh < GEMM_N_SHAPES; ++sh)
+            if (a.tiles[sh].size() != b.tiles[sh].size() ||
+                !std::equal(a.tiles[sh].begin(), a.tiles[sh].end(), b.tiles[sh].begin(), same_tile))
+                return false;
+        return true;
+    };
+    std::vector<GemmCandidate> out;
+    for (int i = 0; i < GEMM_N_POLICIES; ++i) {
+        GemmCandidate c{i, build_gemm_schedule(probs, gemm_policy(i))};
+        bool known = false;
+        for (GemmCandidate const& o : out) known |= same(o.schedule, c.schedule);
+        if (!known) out.push_back(std::move(c));
+    }
+    return out;
+}
+
 uint64_t gemm_stage_key(std::vector<GemmDesc> const& probs) {
     double w = 0, lm = 0, ln = 0, lk = 0, f32 = 0, f64 = 0, f96 = 0, tiles = 0;
     bool rowmap = false;

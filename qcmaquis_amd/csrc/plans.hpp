@@ -240,6 +240,13 @@ inline GemmSchedule build_gemm_schedule(std::vector<GemmDesc> const& probs, int6
     p.min_chunk = min_chunk;
     return build_gemm_schedule(probs, p);
 }
+// the policies whose schedules of a stage differ from each other, the default rule (0) first: stacked
+// problems are never split along K, so a stage of them has that one only
+struct GemmCandidate {
+    int policy;
+    GemmSchedule schedule;
+};
+std::vector<GemmCandidate> gemm_candidates(std::vector<GemmDesc> const& probs);
 // Work item of the device's GEMM kernel: rows [m0, m0 + ml), ml <= 128, and up to 128 columns from n0 of
 // a problem's C (of batch entry `batch`), reduced over [k0, k1); ws < 0: written to C, else the
 // partial tile at element ws of the workspace with leading dimension bm.

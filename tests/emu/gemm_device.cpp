@@ -51,18 +51,32 @@ extern "C" long fold_check(int sym, const mq_mpo_desc* md, const mq_bindex_desc*
     }
 }
 
+// C problems of the given sizes
+static std::vector<GemmDesc> problems(int n, const int* M, const int* N, const int* K, int batch, int flags) {
+    std::vector<GemmDesc> G;
+    for (int i = 0; i < n; ++i) {
+        GemmDesc g{};
+        g.M = M[i];
+        g.N = N[i];
+        g.K = K[i];
+        g.batch = batch;
+        g.flags = flags;
+        G.push_back(g);
+    }
+    return G;
+}
+
+// the policies that the autotuner times for a stage, one bit each
+extern "C" long candidate_policies(int n, const int* M, const int* N, const int* K, int batch, int flags) {
+    long bits = 0;
+    for (GemmCandidate const& c : gemm_candidates(problems(n, M, N, K, batch, flags))) bits |= 1L << c.policy;
+    return bits;
+}
+
 // work items of C problems of the given sizes under schedule candidate `policy`; splits or -1
 extern "C" long items_check(int n, const int* M, const int* N, const int* K, int batch, int policy) {
     try {
-        std::vector<GemmDesc> G;
-        for (int i = 0; i < n; ++i) {
-            GemmDesc g{};
-            g.M = M[i];
-            g.N = N[i];
-            g.K = K[i];
-            g.batch = batch;
-            G.push_back(g);
-        }
+        const std::vector<GemmDesc> G = problems(n, M, N, K, batch, 0);
         const GemmSchedule sch = build_gemm_schedule(G, gemm_policy(policy));
         std::vector<std::vector<int64_t>> done(size_t(n) * batch);
         for (int i = 0; i < n; ++i)

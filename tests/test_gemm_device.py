@@ -27,6 +27,8 @@ def lib():
     ints = C.POINTER(C.c_int)
     lib.items_check.restype = C.c_long
     lib.items_check.argtypes = [C.c_int, ints, ints, ints, C.c_int, C.c_int]
+    lib.candidate_policies.restype = C.c_long
+    lib.candidate_policies.argtypes = [C.c_int, ints, ints, ints, C.c_int, C.c_int]
     return lib
 
 
@@ -61,3 +63,15 @@ def test_work_items(lib, policy):
     k = [1, 17, 256, 1000, 513, 3, 16, 700, 2049, 128, 4000, 31]
     arr = [(C.c_int * len(v))(*v) for v in (m, n, k)]
     assert lib.items_check(len(m), *arr, 2, policy) > 0
+
+
+@pytest.mark.parametrize("flags,batch", [(4, 1), (6, 5), (0, 1)])  # GEMM_ROWMAP, with GEMM_TRANS_B, plain
+def test_autotuner_candidates(lib, flags, batch):
+    """a stage whose schedules are all alike (stacked problems, which K is not split for, and reductions
+    too short to be split) has the default rule only; the others have every schedule once"""
+    arr = lambda *v: (C.c_int * len(v))(*v)
+    long_k = (arr(64, 130, 97), arr(300, 128, 5), arr(9000, 4000, 2049))
+    short_k = (arr(64, 130), arr(300, 128), arr(100, 16))
+    assert lib.candidate_policies(2, *short_k, batch, flags) == 1
+    bits = lib.candidate_policies(3, *long_k, batch, flags)
+    assert bits == 1 if flags & 4 else bits & 1 and bin(bits).count("1") > 2
