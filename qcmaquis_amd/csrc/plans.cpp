@@ -1845,6 +1845,16 @@ GemmPolicy gemm_policy(int i) {
     return p;
 }
 
+// shape and number of the output tiles of a problem: the fewest row tiles, of about equal height
+static int shape_of(GemmDesc const& g) {
+    const int32_t nt = (g.M + 127) / 128, h = (g.M + nt - 1) / nt;
+    return h <= 32 ? GEMM_32 : h <= 64 ? GEMM_64 : h <= 96 ? GEMM_96 : GEMM_128;
+}
+static int64_t tiles_of(GemmDesc const& g) {
+    const int sh = shape_of(g);
+    return int64_t((g.M + gemm_bm(sh) - 1) / gemm_bm(sh)) * ((g.N + gemm_bn(sh) - 1) / gemm_bn(sh)) * g.batch;
+}
+
 std::vector<GemmCandidate> gemm_candidates(std::vector<GemmDesc> const& probs) {
     auto same_tile = [](GemmTile const& a, GemmTile const& b) {
         return a.prob == b.prob && a.batch == b.batch && a.tm == b.tm && a.tn == b.tn && a.k0 == b.k0 && a.k1 == b.k1 &&
@@ -1881,7 +1891,7 @@ uint64_t gemm_stage_key(std::vector<GemmDesc> const& probs) {
         if (g.M <= 32) f32 += f;
         else if (g.M <= 64) f64 += f;
         else if (g.M <= 96) f96 += f;
-        tiles += std::ceil(g.M / 128.0) * std::ceil(g.N / 64.0) * g.batch;
+        tiles += double(tiles_of(g));
         rowmap |= (g.flags & GEMM_ROWMAP) != 0;
     }
     if (w == 0) return 0;
@@ -1905,16 +1915,11 @@ GemmSchedule build_gemm_schedule(std::vector<GemmDesc> const& probs, GemmPolicy 
     const int32_t min_chunk = pol.min_chunk;
     require(min_chunk >= 16 && min_chunk % 16 == 0, "gemm schedule: chunk must be a multiple of 16");
     GemmSchedule S;
-    auto shape_of = [](GemmDesc const& g) {
-        const int32_t nt = (g.M + 127) / 128, h = (g.M + nt - 1) / nt;
-        return h <= 32 ? GEMM_32 : h <= 64 ? GEMM_64 : h <= 96 ? GEMM_96 : GEMM_128;
-    };
     int64_t n_tiles = 0;
     double work = 0;
     for (auto const& g : probs) {
         if (g.M <= 0 || g.N <= 0) continue;
-        const int sh = shape_of(g);
-        const int64_t n = int64_t((g.M + gemm_bm(sh) - 1) / gemm_bm(sh)) * ((g.N + gemm_bn(sh) - 1) / gemm_bn(sh)) * g.batch;
+        const int64_t n = tiles_of(g);
         n_tiles += n;
         work += double(n) * g.K;
     }

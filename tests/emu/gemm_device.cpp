@@ -73,6 +73,13 @@ extern "C" long candidate_policies(int n, const int* M, const int* N, const int*
     return bits;
 }
 
+// the autotuner's key of a stage, and the tiles of its schedule without a split along K
+extern "C" uint64_t stage_key(int n, const int* M, const int* N, const int* K, int batch, long* tiles) {
+    const std::vector<GemmDesc> G = problems(n, M, N, K, batch, 0);
+    *tiles = long(build_gemm_schedule(G, 0, 16).n_tiles());
+    return gemm_stage_key(G);
+}
+
 // work items of C problems of the given sizes under schedule candidate `policy`; splits or -1
 extern "C" long items_check(int n, const int* M, const int* N, const int* K, int batch, int policy) {
     try {

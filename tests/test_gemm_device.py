@@ -1,5 +1,6 @@
 """The device form of the grouped GEMM stages against the plan's own problems, on the CPU."""
 import ctypes as C
+import math
 import os
 import subprocess
 
@@ -29,6 +30,8 @@ def lib():
     lib.items_check.argtypes = [C.c_int, ints, ints, ints, C.c_int, C.c_int]
     lib.candidate_policies.restype = C.c_long
     lib.candidate_policies.argtypes = [C.c_int, ints, ints, ints, C.c_int, C.c_int]
+    lib.stage_key.restype = C.c_uint64
+    lib.stage_key.argtypes = [C.c_int, ints, ints, ints, C.c_int, C.POINTER(C.c_long)]
     return lib
 
 
@@ -75,3 +78,12 @@ def test_autotuner_candidates(lib, flags, batch):
     assert lib.candidate_policies(2, *short_k, batch, flags) == 1
     bits = lib.candidate_policies(3, *long_k, batch, flags)
     assert bits == 1 if flags & 4 else bits & 1 and bin(bits).count("1") > 2
+
+
+@pytest.mark.parametrize("m,n,k", [((128,), (128,), (700,)), ((129,), (64,), (300,)), ((200, 300), (1000, 65), (50, 4000)),
+                                   ((33, 1, 97), (5, 4000, 257), (100, 9, 3))])
+def test_stage_key_counts_tiles(lib, m, n, k):
+    """the tile count in a stage's key (log2, bits 1 to 6) is the one of the schedule"""
+    arr, tiles = [(C.c_int * len(v))(*v) for v in (m, n, k)], C.c_long()
+    key = lib.stage_key(len(m), *arr, 8, C.byref(tiles))
+    assert tiles.value > 0 and (key - 1) >> 1 & 63 == math.floor(math.log2(tiles.value) + 0.5)
