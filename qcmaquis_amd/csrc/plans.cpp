@@ -1819,7 +1819,7 @@ std::vector<GemmDesc> fold_batches(std::vector<GemmDesc> const& v) {
     for (auto& g : out) {
         // C row m, column n of block b at c + (n + b sc) ld: one run of columns when sc is N
         if (g.batch <= 1 || !(g.flags & GEMM_ROWMAP) || !(g.flags & GEMM_TRANS_B) || g.sc != g.N || g.N <= 0 ||
-            int64_t(g.N) * g.batch >= INT32_MAX)
+            int64_t(g.N) * g.batch > INT32_MAX - gemm_bn(0))
             continue;
         g.nb = g.N;
         g.N *= g.batch;

@@ -51,6 +51,21 @@ extern "C" long fold_check(int sym, const mq_mpo_desc* md, const mq_bindex_desc*
     }
 }
 
+// columns of a stacked transposed problem of `batch` blocks of N once folded, and its column tiles as
+// the schedule counts them (32-bit arithmetic)
+extern "C" void fold_columns(int N, int batch, long* columns, long* tiles) {
+    GemmDesc g{};
+    g.M = g.K = 1;
+    g.N = N;
+    g.batch = batch;
+    g.sc = N;
+    g.flags = GEMM_ROWMAP | GEMM_TRANS_B;
+    const GemmDesc f = fold_batches({g})[0];
+    *columns = f.N;
+    const int32_t bn = gemm_bn(0);
+    *tiles = long(int32_t(uint32_t(f.N) + uint32_t(bn) - 1) / bn);
+}
+
 // C problems of the given sizes
 static std::vector<GemmDesc> problems(int n, const int* M, const int* N, const int* K, int batch, int flags) {
     std::vector<GemmDesc> G;

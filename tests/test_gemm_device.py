@@ -32,6 +32,7 @@ def lib():
     lib.candidate_policies.argtypes = [C.c_int, ints, ints, ints, C.c_int, C.c_int]
     lib.stage_key.restype = C.c_uint64
     lib.stage_key.argtypes = [C.c_int, ints, ints, ints, C.c_int, C.POINTER(C.c_long)]
+    lib.fold_columns.argtypes = [C.c_int, C.c_int, C.POINTER(C.c_long), C.POINTER(C.c_long)]
     return lib
 
 
@@ -87,3 +88,12 @@ def test_stage_key_counts_tiles(lib, m, n, k):
     arr, tiles = [(C.c_int * len(v))(*v) for v in (m, n, k)], C.c_long()
     key = lib.stage_key(len(m), *arr, 8, C.byref(tiles))
     assert tiles.value > 0 and (key - 1) >> 1 & 63 == math.floor(math.log2(tiles.value) + 0.5)
+
+
+@pytest.mark.parametrize("n,batch,fold", [(5, 7, True), (16777215, 128, False), (1073741821, 2, False),
+                                          (67108863, 32, False), (65535, 32766, True)])
+def test_folded_columns_fit(lib, n, batch, fold):
+    """blocks are folded only while the rounded-up column count is a 32-bit number"""
+    cols, tiles = C.c_long(), C.c_long()
+    lib.fold_columns(n, batch, C.byref(cols), C.byref(tiles))
+    assert cols.value == (n * batch if fold else n) and tiles.value == -(-cols.value // 128)
