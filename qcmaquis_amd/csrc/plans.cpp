@@ -1727,56 +1727,51 @@ void check_sblocks(SBlockTable const& B, uint64_t t_size, uint64_t s_size) {
                 bad = std::max(bad, 3);
         }
     }
-    // every element range of every block in exactly one work item (in any order)
+    // every element range of every block in exactly one work item (in any order), and every work item
+    // in exactly one launch entry
     if (bad == 0) {
         std::vector<uint64_t> first(B.blocks.size() + 1, 0);
         for (size_t bi = 0; bi < B.blocks.size(); ++bi)
             first[bi + 1] = first[bi] + uint64_t((B.blocks[bi].E + SBLOCK_ELEMS - 1) / SBLOCK_ELEMS);
-        std::vector<char> seen(first.back(), 0);
+        std::vector<char> seen(first.back(), 0), dealt(first.back(), 0);
         if (B.work.size() != first.back() || B.n_work.team < 0 || B.n_work.pair < 0 || B.n_work.solo < 0 ||
             uint64_t(B.n_work.team) + uint64_t(B.n_work.pair) + uint64_t(B.n_work.solo) != B.work.size())
             bad = std::max(bad, 4);
-        for (size_t i = 0; i < B.work.size(); ++i) {
-            SWork const& w = B.work[i];
+        auto mark = [&](SWork const& w, std::vector<char>& v) {
             if (!(w.blk >= 0 && size_t(w.blk) < B.blocks.size() && w.n0 >= 0 && w.n0 < B.blocks[size_t(w.blk)].E &&
                   w.n0 % SBLOCK_ELEMS == 0)) {
                 bad = std::max(bad, 4);
-                continue;
+                return;
             }
-            // an item of fewer waves than its tile needs would leave elements unwritten
-            const int32_t E = B.blocks[size_t(w.blk)].E;
-            if (i >= size_t(B.n_work.team) && (E > 64 || (i >= size_t(B.n_work.team) + size_t(B.n_work.pair) && E > 32)))
-                bad = std::max(bad, 4);
-            char& c = seen[first[size_t(w.blk)] + uint64_t(w.n0 / SBLOCK_ELEMS)];
+            char& c = v[first[size_t(w.blk)] + uint64_t(w.n0 / SBLOCK_ELEMS)];
             if (c) bad = std::max(bad, 4);
             c = 1;
-        }
-    }
-    // every work item in exactly one launch entry
-    if (bad == 0) {
+        };
+        for (SWork const& w : B.work) mark(w, seen);
         const int64_t nt = B.n_work.team, np = B.n_work.pair, n = int64_t(B.work.size());
-        uint64_t teams = 0, items = 0;
-        std::vector<char> small(size_t(n - nt), 0);
-        for (SWork const& l : B.launch) {
+        // an item of fewer waves than its tile needs would leave elements unwritten
+        for (int64_t i = 0; bad == 0 && i < n; ++i) {
+            const int32_t E = B.blocks[size_t(B.work[size_t(i)].blk)].E;
+            if (i < nt ? E <= 64 : i < nt + np ? E <= 32 || E > 64 : E > 32) bad = 4;
+        }
+        uint64_t dealt_n = 0;
+        for (size_t q = 0; bad == 0 && q < B.launch.size(); ++q) {
+            SWork const& l = B.launch[q];
             if (l.blk >= 0) {
-                ++teams;
-                if (size_t(l.blk) >= B.blocks.size() || B.blocks[size_t(l.blk)].E <= 64 || l.n0 < 0 ||
-                    l.n0 >= B.blocks[size_t(l.blk)].E || l.n0 % SBLOCK_ELEMS != 0)
-                    bad = std::max(bad, 4);
+                mark(l, dealt);
+                if (bad == 0 && B.blocks[size_t(l.blk)].E <= 64) bad = 4;
+                ++dealt_n;
                 continue;
             }
             const int64_t waves = l.blk < -2 ? -int64_t(l.blk) - 2 : -l.blk, per = l.blk < -2 ? 1 : SB_WAVES / waves;
             const int64_t lo = waves == 1 ? nt + np : nt, hi = waves == 1 ? n : nt + np;
             if (waves > 2 || l.n0 < lo || l.n0 >= hi) {
-                bad = std::max(bad, 4);
+                bad = 4;
                 continue;
             }
-            for (int64_t i = l.n0; i < std::min<int64_t>(hi, l.n0 + per); ++i, ++items) {
-                if (small[size_t(i - nt)]) bad = std::max(bad, 4);
-                small[size_t(i - nt)] = 1;
-            }
+            for (int64_t i = l.n0; i < std::min<int64_t>(hi, l.n0 + per); ++i, ++dealt_n) mark(B.work[size_t(i)], dealt);
         }
-        if (teams != uint64_t(nt) || items != uint64_t(n - nt)) bad = std::max(bad, 4);
+        if (dealt_n != uint64_t(n)) bad = std::max(bad, 4);
     }
     // small-tile tables: 5 malformed line, 6 term tile outside T, 7 malformed work item
     const int64_t nsl = int64_t(B.small_lines.size());

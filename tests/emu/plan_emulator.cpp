@@ -191,6 +191,40 @@ struct EmuBoundary {
 extern "C" {
 
 void emu_set_sblock_panel(int panel) { g_panel = panel; }
+// check_sblocks on a launch list with entry `to` replaced by a copy of entry `from` (none when `from` < 0),
+// of 200 lines each of 1, 30, 64, 100, 300 and 700 elements that read `tiles` T tiles: 1 accepted, 0 rejected;
+// from, to count the entries whose blk is `kind`, or any blk >= 0 when `kind` is 0
+int emu_launch_copied(int tiles, int kind, int from, int to) {
+    HostTable<SLine> lines;
+    HostTable<STerm> terms;
+    int64_t s_off = 0;
+    for (int E : {1, 30, 64, 100, 300, 700})
+        for (int l = 0; l < 200; ++l) {
+            SLine q{};
+            q.s_off = s_off;
+            s_off += E;
+            q.rows = q.lds = E;
+            q.cols = 1;
+            q.t0 = int32_t(terms.size());
+            for (int t = 0; t < tiles; ++t) terms.push_back(STerm{1.0, 700 * int64_t(t)});
+            q.t1 = int32_t(terms.size());
+            lines.push_back(q);
+        }
+    try {
+        SBlockTable B = build_sblocks(lines, terms, 0);
+        std::vector<size_t> e;
+        for (size_t i = 0; i < B.launch.size(); ++i)
+            if (kind == 0 ? B.launch[i].blk >= 0 : B.launch[i].blk == kind) e.push_back(i);
+        if (from >= 0) B.launch.at(e.at(size_t(to))) = B.launch.at(e.at(size_t(from)));
+        check_sblocks(B, 700 * uint64_t(tiles), uint64_t(s_off));
+        return 1;
+    } catch (Error const&) {
+        return 0;
+    } catch (std::exception const& e) {
+        fprintf(stderr, "emu_launch_copied: %s\n", e.what());
+        return -1;
+    }
+}
 void emu_set_gemm_policy(int policy) { g_policy = policy; }
 
 int emu_hpsi(int sym, const mq_mpo_desc* md, const mq_bindex_desc* Ld, const double* Ldata, const mq_bindex_desc* Rd,

@@ -96,3 +96,14 @@ def test_nonsymmetric_left(oracle_lib):
                               symmetric=False)
         same_index(Le, Lo)
         assert rel_err(Le.data, Lo.data) < 1e-12
+
+
+# (tiles a line reads, kind of launch entry, entry copied, entry lost): team items (0) of other ranges and of other
+# blocks, workgroups of two-wave and of one-wave items (-2, -1), and with their k-steps shared out (-4, -3)
+@pytest.mark.parametrize("tiles,kind,src,dst", [(5, 0, 0, 1), (5, 0, 3, 2), (5, 0, 5, 20), (5, -2, 0, 1), (5, -1, 1, 0),
+                                                (300, 0, 7, 1), (300, -4, 0, 1), (300, -3, 2, 0)])
+def test_launch_list_with_an_entry_lost(tiles, kind, src, dst):
+    """a launch list that deals one work item twice in place of another is rejected"""
+    f = emu.lib().emu_launch_copied
+    assert f(tiles, kind, -1, 0) == 1 and f(tiles, kind, src, src) == 1
+    assert f(tiles, kind, src, dst) == 0
