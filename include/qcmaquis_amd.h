@@ -66,7 +66,10 @@ extern "C" {
                                   element, instead of in 16-tile blocks on the matrix cores (0: every
                                   tile in blocks); MQ_SMALL_TILE_AUTO (default): per site problem,
                                   64 when its mean S tile has at most 16 elements and the plan at
-                                  most 2^19 terms, else 0 */
+                                  most 2^19 terms, else 0.  The two forms round differently.  A
+                                  non-finite element of T reaches the lines that read its tile; in
+                                  tiles of more than 64 elements, always summed in blocks by the
+                                  automatic rule, also the other lines of their block */
 #define MQ_SMALL_TILE_AUTO (-1)
 #define MQ_OPT_CHUNK_MB 3      /* value >= 0: H*psi plans made afterwards split their output columns
                                   by right sector into chunks of at most this many MiB of FP64 T and

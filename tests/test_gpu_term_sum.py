@@ -15,20 +15,28 @@ from tests.chains import oracle_left, oracle_right, rel_err
 pytestmark = pytest.mark.gpu
 
 
-def run(oracle_lib, ctx, s, D, small_max):
+def problem(oracle_lib, s, D):
     ch = Chain(np.random.default_rng(100 + s), abi.MQ_SYM_TWOU1, 4, (4, 4), s, D,
                phys=fuse_index(TWOU1_SITE, TWOU1_SITE), density=0.5, min_m=s)
     k = 2
     L = oracle_left(oracle_lib, ch, k)[k]
     R = oracle_right(oracle_lib, ch, k + 1)[k + 1]
     lay = ch.layouts[k]
-    psi = np.random.default_rng(s).normal(size=lay.n)
-    ref = oracle_lib.hpsi(ch.sym, ch.mpos[k], L, R, lay, psi)
+    return ch.sym, ch.mpos[k], L, R, lay, np.random.default_rng(s).normal(size=lay.n)
+
+
+def make_plan(ctx, mpo, L, R, lay, small_max):
     ctx.set_option(abi.MQ_OPT_SMALL_TILE_MAX, small_max)
     try:
-        plan = HpsiPlan(ctx, DeviceMPO(ctx, ch.mpos[k]), DeviceBoundary.upload(ctx, L), DeviceBoundary.upload(ctx, R), lay)
+        return HpsiPlan(ctx, DeviceMPO(ctx, mpo), DeviceBoundary.upload(ctx, L), DeviceBoundary.upload(ctx, R), lay)
     finally:
         ctx.set_option(abi.MQ_OPT_SMALL_TILE_MAX, abi.MQ_SMALL_TILE_AUTO)
+
+
+def run(oracle_lib, ctx, s, D, small_max):
+    sym, mpo, L, R, lay, psi = problem(oracle_lib, s, D)
+    ref = oracle_lib.hpsi(sym, mpo, L, R, lay, psi)
+    plan = make_plan(ctx, mpo, L, R, lay, small_max)
     st = plan.stats()
     err = rel_err(plan.apply(psi), ref)
     err32 = rel_err(plan.apply(psi, abi.MQ_PREC_FP32), ref)
@@ -51,3 +59,26 @@ def test_small_line_groups(oracle_lib, ctx2u1, s, D):
     st, err, err32 = run(oracle_lib, ctx2u1, s, D, 256)  # every tile term by term
     assert st["n_sblocks"] == 0 and st["small_lines"] > 0
     assert err < 1e-12 and err32 < 1e-5
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("s,D", [(1, 24), (5, 24), (8, 24), (1, 64), (6, 64)])
+def test_non_finite_elements(oracle_lib, ctx2u1, s, D, value):
+    """an infinite or undefined psi element reaches the same elements of H*psi whether tiles of at most 64
+    elements are summed in blocks or term by term, i.e. only those whose lines read it; the others agree to
+    1e-12 (FP64) and 1e-5 (FP32) of the largest of them"""
+    sym, mpo, L, R, lay, psi = problem(oracle_lib, s, D)
+    plans = [make_plan(ctx2u1, mpo, L, R, lay, m) for m in (256, 0)]
+    few = 0
+    for at in (0, lay.n // 2, lay.n - 1):
+        x = psi.copy()
+        x[at] = value
+        for prec, tol in ((abi.MQ_PREC_FP64, 1e-12), (abi.MQ_PREC_FP32, 1e-5)):
+            terms, blocks = (p.apply(x, prec) for p in plans)
+            ok = np.isfinite(terms)
+            print(f"tiles {s}x{s}, psi[{at}] = {value}: {ok.sum()} of {lay.n} finite, in blocks {np.isfinite(blocks).sum()}",
+                  flush=True)
+            assert np.array_equal(ok, np.isfinite(blocks))
+            assert not ok.any() or rel_err(blocks[ok], terms[ok]) < tol
+            few += 0 < ok.sum() < lay.n
+    assert few > 0
