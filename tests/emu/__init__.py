@@ -34,6 +34,7 @@ def lib():
                                C.c_int, P(C.c_uint64), C.c_uint64, P(C.c_uint64), P(C.c_uint64), C.c_int]
         L.emu_set_sblock_panel.argtypes = [C.c_int]
         L.emu_set_gemm_policy.argtypes = [C.c_int]
+        L.emu_shared_items.restype = C.c_long
         L.emu_term_grad.argtypes = [C.c_int, P(abi.MPODesc), P(abi.BIndexDesc), dp, P(abi.BIndexDesc), dp, idx, idx,
                                     idx, dp, dp, C.c_uint64]
         for f in (L.emu_lstep, L.emu_rstep):

@@ -16,52 +16,50 @@ using namespace mq;
 
 namespace {
 
-// executes the stage as the device does: the tiles of the GEMM schedule, each over its K range,
-// writing C or a workspace partial, then the split-K reduce jobs.  The schedule is built with a
-// K chunk of 16 so that every reduction longer than one K slice goes through the split path.
+// executes the stage as the device does: its problems with folded batches, the work items of the GEMM
+// schedule, each over its K range, writing C or a workspace partial, then the split-K reduce jobs.  The
+// schedule is built with a K chunk of 16 so that every reduction longer than one K slice goes through
+// the split path.
 // GEMM schedule: < 0 every reduction longer than one K slice split (below), else the autotuner's
 // candidate of that index
 int g_policy = -1;
 
-void run_gemms(std::vector<GemmDesc> const& G, std::vector<GemmRow> const& rows, double* const* base) {
+void run_gemms(std::vector<GemmDesc> const& stage, std::vector<GemmRow> const& rows, double* const* base) {
+    const std::vector<GemmDesc> G = fold_batches(stage);
     GemmSchedule sch = g_policy < 0 ? build_gemm_schedule(G, int64_t(1) << 40, 16)
                                     : build_gemm_schedule(G, gemm_policy(g_policy));
     std::vector<double> ws(sch.ws_elems + 1, std::nan(""));
     std::vector<char> seen(sch.ws_elems + 1, 0);
-    for (int sh = 0; sh < GEMM_N_SHAPES; ++sh) {
-        const int bm = gemm_bm(sh), bn = gemm_bn(sh);
-        for (GemmTile const& t : sch.tiles[sh]) {
-            GemmDesc const& g = G[t.prob];
-            bool ta = g.flags & GEMM_TRANS_A, tb = g.flags & GEMM_TRANS_B, rmap = g.flags & GEMM_ROWMAP;
-            require(!rmap || t.ws < 0, "emulated gemm: stacked problem split along K");
-            const double* A = base[g.base_a] + (rmap ? 0 : g.a + int64_t(t.batch) * g.sa);
-            const double* B = base[g.base_b] + g.b + int64_t(t.batch) * g.sb;
-            double* Cm = base[g.base_c] + (rmap ? 0 : g.c + int64_t(t.batch) * g.sc);
-            for (int nn = 0; nn < bn; ++nn)
-                for (int mm = 0; mm < bm; ++mm) {
-                    int m = t.tm * bm + mm, n = t.tn * bn + nn;
-                    if (m >= g.M || n >= g.N) continue;
-                    GemmRow row{};
-                    if (rmap) row = rows.at(size_t(g.a + m));
-                    double s = 0.0;
-                    for (int k = t.k0; k < t.k1; ++k) {
-                        double a = rmap ? A[row.a + int64_t(k) * row.ld]
-                                        : ta ? A[int64_t(m) * g.lda + k] : A[m + int64_t(k) * g.lda];
-                        double v = tb ? B[n + int64_t(k) * g.ldb] : B[k + int64_t(n) * g.ldb];
-                        s += a * v;
-                    }
-                    if (rmap) {
-                        Cm[row.c + (n + int64_t(t.batch) * g.sc) * row.ld] = s;
-                    } else if (t.ws < 0) {
-                        Cm[m + int64_t(n) * g.ldc] = s;
-                    } else {
-                        uint64_t w = uint64_t(t.ws) + mm + uint64_t(nn) * bm;
-                        require(w < sch.ws_elems && !seen[w], "emulated gemm: workspace slot out of range or reused");
-                        seen[w] = 1;
-                        ws[w] = s;
-                    }
+    for (GemmItem const& t : gemm_items(G, sch)) {
+        GemmDesc const& g = G.at(size_t(t.prob));
+        bool ta = g.flags & GEMM_TRANS_A, tb = g.flags & GEMM_TRANS_B, rmap = g.flags & GEMM_ROWMAP;
+        require(!rmap || t.ws < 0, "emulated gemm: stacked problem split along K");
+        const double* A = base[g.base_a] + (rmap ? 0 : g.a + int64_t(t.batch) * g.sa);
+        const double* B = base[g.base_b] + g.b + int64_t(t.batch) * g.sb;
+        double* Cm = base[g.base_c] + (rmap ? 0 : g.c + int64_t(t.batch) * g.sc);
+        for (int nn = 0; nn < std::min(128, g.N - t.n0); ++nn)
+            for (int mm = 0; mm < t.ml; ++mm) {
+                const int m = t.m0 + mm, n = t.n0 + nn;
+                GemmRow row{};
+                if (rmap) row = rows.at(size_t(g.a + m));
+                const int64_t bn = g.flags & GEMM_NBLOCKS ? int64_t(n / g.nb) * g.sb + n % g.nb : n;
+                double s = 0.0;
+                for (int k = t.k0; k < t.k1; ++k) {
+                    double a = rmap ? A[row.a + int64_t(k) * row.ld]
+                                    : ta ? A[int64_t(m) * g.lda + k] : A[m + int64_t(k) * g.lda];
+                    s += a * (tb ? B[bn + int64_t(k) * g.ldb] : B[k + int64_t(n) * g.ldb]);
                 }
-        }
+                if (rmap) {
+                    Cm[row.c + (n + int64_t(t.batch) * g.sc) * row.ld] = s;
+                } else if (t.ws < 0) {
+                    Cm[m + int64_t(n) * g.ldc] = s;
+                } else {
+                    uint64_t w = uint64_t(t.ws) + mm + uint64_t(nn) * t.bm;
+                    require(w < sch.ws_elems && !seen[w], "emulated gemm: workspace slot out of range or reused");
+                    seen[w] = 1;
+                    ws[w] = s;
+                }
+            }
     }
     for (GemmReduce const& r : sch.reduces) {
         GemmDesc const& g = G[r.prob];
@@ -82,14 +80,17 @@ void run_gemms(std::vector<GemmDesc> const& G, std::vector<GemmRow> const& rows,
     }
 }
 
-// the MPO-term sum as the device runs it: the block table built from the lines, each work item
-// covering SBLOCK_ELEMS tile elements of one block, the groups of 16 lines summing the sub-blocks of
-// the k-steps their masks name; every (line, element) of the table must be written exactly once
-// (tiles of at most small_max elements: the small-tile work items, 2^lg lanes per line, lane e
-// summing element e over the line's terms)
+// the MPO-term sum as the device runs it: the block table built from the lines, the entries of its launch
+// list one workgroup each -- a block's range of SBLOCK_ELEMS tile elements, or the items of smaller tiles
+// that share a workgroup, or one of them with its k-steps in equal shares summed pairwise --, the groups
+// of 16 lines summing the sub-blocks of the k-steps their masks name; every (line, element) of the table
+// must be written exactly once (tiles of at most small_max elements: the small-tile work items, 2^ts
+// shares of a line's terms of 2^lg lanes, lane e summing element e)
 // Returns the number of small-tile lines.
 // panel of the term-sum work order (MQ_OPT_SBLOCK_PANEL; the product's automatic value by default)
 int32_t g_panel = 16;
+// workgroups that shared out the k-steps of one item so far
+long g_shared = 0;
 
 uint64_t run_lines(HostTable<SLine>& lines, HostTable<STerm> const& terms, const double* T, double* S,
                    uint64_t t_size, uint64_t s_size, int32_t small_max = 0) {
@@ -101,12 +102,14 @@ uint64_t run_lines(HostTable<SLine>& lines, HostTable<STerm> const& terms, const
     uint64_t small_covered = 0;
     for (SSmallWork const& w : B.small_work)
         for (int lane = 0; lane < SMALL_LINE_LANES; ++lane) {
-            const int li = lane >> w.lg, e = lane & ((1 << w.lg) - 1);
+            const int li = lane >> (w.lg + w.ts), e = lane & ((1 << w.lg) - 1), share = (lane >> w.lg) & ((1 << w.ts) - 1);
             if (li >= w.n) continue;
             SLine const& l = B.small_lines[size_t(w.line0 + li)];
-            if (e >= l.rows * l.cols) continue;
+            if (e >= l.rows * l.cols || share > 0) continue;  // the sums of the shares meet in the first
             double acc = 0.0;
-            for (int32_t k = l.t0; k < l.t1; ++k) acc += B.small_terms[size_t(k)].alpha * T[B.small_terms[size_t(k)].t_off + e];
+            for (int q = 0; q < 1 << w.ts; ++q)
+                for (int32_t k = l.t0 + q; k < l.t1; k += 1 << w.ts)
+                    acc += B.small_terms[size_t(k)].alpha * T[B.small_terms[size_t(k)].t_off + e];
             S[l.s_off + e % l.rows + int64_t(e / l.rows) * l.lds] = acc;
             if (e == 0) {
                 require(!sdone[size_t(w.line0 + li)], "emulated small lines: line written twice");
@@ -117,32 +120,51 @@ uint64_t run_lines(HostTable<SLine>& lines, HostTable<STerm> const& terms, const
     for (char d : sdone) require(d, "emulated small lines: line not written");
     std::vector<std::vector<char>> done(B.blocks.size());
     for (size_t i = 0; i < B.blocks.size(); ++i) done[i].assign(size_t(B.blocks[i].E) * SBLOCK_LINES, 0);
-    for (SWork const& w : B.work) {
-        SBlock const& b = B.blocks[size_t(w.blk)];
-        for (int e = w.n0; e < std::min(b.E, w.n0 + SBLOCK_ELEMS); ++e) {
+    // elements [w.n0, w.n0 + elems) of an item's block, its k-steps in `parts` shares
+    auto run_item = [&](SWork const& w, int elems, int parts) {
+        SBlock const& b = B.blocks.at(size_t(w.blk));
+        for (int e = w.n0; e < std::min(b.E, w.n0 + elems); ++e) {
             // the k-steps in order, each group with a sub-block adding alpha_g(16 x 4) * X(4 tiles)
-            double acc[SBLOCK_LINES] = {0.0};
-            for (int32_t k = 0; k < b.nk; ++k) {
-                const uint32_t word = B.kstep[size_t(b.k_off + k)];
-                int64_t ai = b.a_off + int64_t(word >> 8);
-                for (int g = 0; g < SBLOCK_GROUPS; ++g) {
-                    if (!((word >> g) & 1u)) continue;
-                    for (int t = 0; t < 4; ++t) {
-                        const int64_t to = B.utile[size_t(4 * int64_t(b.k_off + k) + t)];
-                        const double x = to >= 0 ? T[to + e] : 0.0;
-                        for (int i = 0; i < SBLOCK_GROUP; ++i)
-                            acc[g * SBLOCK_GROUP + i] += B.ualpha[size_t(64 * ai + 16 * t + i)] * x;
+            std::vector<std::vector<double>> acc(size_t(parts), std::vector<double>(SBLOCK_LINES, 0.0));
+            for (int p = 0; p < parts; ++p)
+                for (int32_t k = b.nk * p / parts; k < b.nk * (p + 1) / parts; ++k) {
+                    const uint32_t word = B.kstep[size_t(b.k_off + k)];
+                    int64_t ai = b.a_off + int64_t(word >> 8);
+                    for (int g = 0; g < SBLOCK_GROUPS; ++g) {
+                        if (!((word >> g) & 1u)) continue;
+                        for (int t = 0; t < 4; ++t) {
+                            const int64_t to = B.utile[size_t(4 * int64_t(b.k_off + k) + t)];
+                            const double x = to >= 0 ? T[to + e] : 0.0;
+                            for (int i = 0; i < SBLOCK_GROUP; ++i)
+                                acc[size_t(p)][size_t(g * SBLOCK_GROUP + i)] += B.ualpha[size_t(64 * ai + 16 * t + i)] * x;
+                        }
+                        ++ai;
                     }
-                    ++ai;
                 }
-            }
+            for (int h = parts / 2; h > 0; h /= 2)
+                for (int p = 0; p < h; ++p)
+                    for (int i = 0; i < SBLOCK_LINES; ++i) acc[size_t(p)][size_t(i)] += acc[size_t(p + h)][size_t(i)];
             for (int i = 0; i < b.nlines; ++i) {
                 char& d = done[size_t(w.blk)][size_t(e) * SBLOCK_LINES + i];
                 require(!d, "emulated S blocks: element written twice");
                 d = 1;
-                S[B.lsoff[size_t(b.line0 + i)] + e % b.rows + int64_t(e / b.rows) * B.llds[size_t(b.line0 + i)]] = acc[i];
+                S[B.lsoff[size_t(b.line0 + i)] + e % b.rows + int64_t(e / b.rows) * B.llds[size_t(b.line0 + i)]] =
+                    acc[0][size_t(i)];
             }
         }
+    };
+    for (SWork const& l : B.launch) {
+        if (l.blk >= 0) {
+            run_item(l, SBLOCK_ELEMS, 1);
+            continue;
+        }
+        // waves of an item, 32 elements each; the items end with the kind
+        const bool shared = l.blk < -2;
+        const int waves = shared ? -l.blk - 2 : -l.blk;
+        const int64_t end = waves == 2 ? B.n_work.team + B.n_work.pair : int64_t(B.work.size());
+        for (int64_t i = l.n0; i < std::min<int64_t>(end, l.n0 + (shared ? 1 : SB_WAVES / waves)); ++i)
+            run_item(B.work.at(size_t(i)), 32 * waves, shared ? SB_WAVES / waves : 1);
+        g_shared += shared;
     }
     for (size_t i = 0; i < B.blocks.size(); ++i)
         for (int e = 0; e < B.blocks[i].E; ++e)
@@ -225,6 +247,7 @@ int emu_launch_copied(int tiles, int kind, int from, int to) {
         return -1;
     }
 }
+long emu_shared_items() { return g_shared; }
 void emu_set_gemm_policy(int policy) { g_policy = policy; }
 
 int emu_hpsi(int sym, const mq_mpo_desc* md, const mq_bindex_desc* Ld, const double* Ldata, const mq_bindex_desc* Rd,

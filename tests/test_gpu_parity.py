@@ -90,7 +90,7 @@ def test_fp32_hpsi(ctx2u1, ctxsu2, oracle_lib, sym):
     max-norm relative error against the FP64 oracle below 1e-5 (FP32 rounding of psi, L, R, T
     and S with K-long FP32 sums); the split-BF16 products (MQ_PREC_BF16X3: each FP32 operand as
     hi + lo BF16 parts, |x - hi - lo| <= 2^-16 |x|, lo lo left out, so about 3 * 2^-16 per
-    product) below 5e-4, over sector dims 1..90 (ragged K, every tile shape)"""
+    product) below 5e-4, over sector dims 1..90 (ragged K; the tiles' edges beyond: test_gpu_gemm_tiles.py)"""
     from qcmaquis_amd.synthetic import TWOU1_SITE, fuse_index
     ctx = ctx2u1 if sym == abi.MQ_SYM_TWOU1 else ctxsu2
     print(f"fp32 hpsi sym={sym}", flush=True)

@@ -7,9 +7,9 @@ import pytest
 
 from qcmaquis_amd import abi
 from qcmaquis_amd.model import initial_boundary
-from qcmaquis_amd.synthetic import TWOU1_SITE, fuse_index
+from qcmaquis_amd.synthetic import TWOU1_SITE, Chain, fuse_index
 from tests import emu
-from tests.chains import make_chain, rel_err, same_index
+from tests.chains import make_chain, oracle_left, oracle_right, rel_err, same_index
 
 CASES = [
     (abi.MQ_SYM_TWOU1, 1, dict(n_sites=5, total=(3, 2), max_m=3, D=6)),
@@ -96,6 +96,22 @@ def test_nonsymmetric_left(oracle_lib):
                               symmetric=False)
         same_index(Le, Lo)
         assert rel_err(Le.data, Lo.data) < 1e-12
+
+
+@pytest.mark.parametrize("s", [1, 5, 6, 8, 9])  # the chains of tests/test_gpu_term_sum.py
+def test_launch_list_of_long_blocks(oracle_lib, s):
+    """blocks of more k-steps than one workgroup leaves to one wave, on tiles of one wave, of two and of a
+    workgroup: the launch list as the device walks it, all tiles in blocks and term by term"""
+    ch = Chain(np.random.default_rng(100 + s), abi.MQ_SYM_TWOU1, 4, (4, 4), s, 64,
+               phys=fuse_index(TWOU1_SITE, TWOU1_SITE), density=0.5, min_m=s)
+    L, R = oracle_left(oracle_lib, ch, 2)[2], oracle_right(oracle_lib, ch, 3)[3]
+    lay = ch.layouts[2]
+    psi = np.random.default_rng(s).normal(size=lay.n)
+    ref = oracle_lib.hpsi(ch.sym, ch.mpos[2], L, R, lay, psi)
+    before = emu.lib().emu_shared_items()
+    assert rel_err(emu.hpsi(ch.sym, ch.mpos[2], L, R, lay, psi, 0), ref) < 1e-12
+    assert (emu.lib().emu_shared_items() > before) == (s <= 8)
+    assert rel_err(emu.hpsi(ch.sym, ch.mpos[2], L, R, lay, psi, 256), ref) < 1e-12
 
 
 # (tiles a line reads, kind of launch entry, entry copied, entry lost): team items (0) of other ranges and of other
