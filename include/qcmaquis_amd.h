@@ -66,7 +66,8 @@ extern "C" {
                                   element, instead of in 16-tile blocks on the matrix cores (0: every
                                   tile in blocks); MQ_SMALL_TILE_AUTO (default): per site problem,
                                   64 when its mean S tile has at most 16 elements and the plan at
-                                  most 2^19 terms, else 0.  The two forms round differently.  A
+                                  most 2^19 terms (all problems of a batch counted), else 0.  The
+                                  two forms round differently.  A
                                   non-finite element of T reaches the lines that read its tile; in
                                   tiles of more than 64 elements, always summed in blocks by the
                                   automatic rule, also the other lines of their block */

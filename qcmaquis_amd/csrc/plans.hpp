@@ -274,9 +274,15 @@ uint64_t gemm_stage_key(std::vector<GemmDesc> const& probs);
 SBlockTable build_sblocks(HostTable<SLine> const& lines, HostTable<STerm> const& terms, int32_t panel = 0);
 // small-tile limit of the lines [l0, l1) of one site problem under the automatic rule: 64 when
 // their mean tile has at most 16 elements and the plan at most SMALL_TERMS_MAX terms (n_terms; 0:
-// those of the lines count), else 0.  Then the blocks are too few to fill the device: 8 orbitals and
-// M = 40 (0.2 million terms) take 10.5 us term by term, 30 in blocks; 12 and M = 96 (2.0 million)
-// 103 and 65, 18 and M = 128 (21 million) 496 and 252, as a block reads a tile once for 64 lines
+// those of the lines count), else 0.  Term by term every term fetches its tile; a block reads it once
+// for 64 lines, but each has its chain of tables, tiles and matrix cores, some 30 us with few blocks.
+// FP64 term sum in us, term by term / in blocks: 8 orbitals and M = 40 (0.2 million terms) 10.5 / 29, 9
+// and 60 (0.35) 23 / 40, 12 and 96 (2.2) 101 / 59, 18 and 128 (21) 488 / 253.  The line is on the safe
+// side for the blocks: between 0.4 and 5 million terms those win where some tiles have more than 64
+// elements and go to blocks anyway (10 and M = 70, 0.76 million, 68 / 45; 11 and 80, 1.2, 95 / 66), and
+// the terms where none has (10 and M = 45 23 / 39; 12 and 60, 2.2, 34 / 46; 14 and 50, 5.3, 38 / 54).
+// n_terms are those of all problems of a batch, so one of them may be summed in the other form, and
+// rounded otherwise, than in a plan of its own
 constexpr uint64_t SMALL_TERMS_MAX = 1u << 19;
 int32_t auto_small_tile_max(HostTable<SLine> const& lines, size_t l0, size_t l1, uint64_t n_terms = 0);
 // marks the lines [l0, l1) whose tiles have 1 .. limit elements SLINE_SMALL (limit <= 256)
