@@ -555,12 +555,16 @@ __global__ __launch_bounds__(SB_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 // Small-tile MPO-term sum: a work item is up to 256 >> (lg + ts) lines of 2^ts shares of 2^lg lanes
 // (tile elements <= 2^lg); lane e of share s sums alpha_k * T[t_off_k + e] over the line's terms
 // k = s, s + 2^ts, ..., four at a time, the shares are added by lane exchanges (between waves: through
-// LDS), and element e of the line's S tile is written once.  Past its last term a lane reads that
-// term again and leaves it out.
+// LDS), and element e of the line's S tile is written once.  Past its last term a lane of a share reads
+// that term again and leaves it out; a line of one share has few terms or a tile of many elements, and
+// its last terms are read one by one.
 //
 // Bound: the chain terms -> tile elements in the few, small problems that come here (most lines have
 // one or two terms, the longest hundreds).  One lane per element for all of a line's terms, as
-// before, took 24 us for 8 orbitals and M = 40; with a line's terms shared out 10.5.
+// before, took 24 us for 8 orbitals and M = 40; with a line's terms shared out 10.2.  Where a caller
+// sends large problems here the fetches of tiles bound it, and what a lane reads in vain counts: 18
+// orbitals and M = 300, tiles up to 256 elements, 1.17 ms; lines in neighbours' order and every line's last
+// terms read again 1.26, in the order of their term count 1.19, the last terms one by one 1.16.
 template <class T>
 __global__ __launch_bounds__(SMALL_LINE_LANES) void small_lines_kernel(const SSmallWork* __restrict__ work,
                                                                        const SLine* __restrict__ lines,
@@ -576,20 +580,35 @@ __global__ __launch_bounds__(SMALL_LINE_LANES) void small_lines_kernel(const SSm
     if (in) {
         constexpr int U = SMALL_LINE_DEPTH;
         const int last = l.t1 - 1;
-        for (int k = l.t0 + (q >> w.lg); k < l.t1; k += U << w.ts) {
-            STerm t[U];
+        if (w.ts == 0) {
+            int k = l.t0;
+            for (; k + U <= l.t1; k += U) {
+                STerm t[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int ku = k + (u << w.ts);
-                t[u] = terms[ku < last ? ku : last];
+                for (int u = 0; u < U; ++u) t[u] = terms[k + u];
+                T x[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) x[u] = X[t[u].t_off + e];
+#pragma unroll
+                for (int u = 0; u < U; ++u) acc += T(t[u].alpha) * x[u];
             }
-            T x[U];
+            for (; k < l.t1; ++k) acc += T(terms[k].alpha) * X[terms[k].t_off + e];
+        } else {
+            for (int k = l.t0 + (q >> w.lg); k < l.t1; k += U << w.ts) {
+                STerm t[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) x[u] = X[t[u].t_off + e];
+                for (int u = 0; u < U; ++u) {
+                    const int ku = k + (u << w.ts);
+                    t[u] = terms[ku < last ? ku : last];
+                }
+                T x[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const bool ok = k + (u << w.ts) <= last;
-                acc += ok ? T(t[u].alpha) * x[u] : T(0);
+                for (int u = 0; u < U; ++u) x[u] = X[t[u].t_off + e];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const bool ok = k + (u << w.ts) <= last;
+                    acc += ok ? T(t[u].alpha) * x[u] : T(0);
+                }
             }
         }
     }

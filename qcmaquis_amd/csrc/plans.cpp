@@ -1376,7 +1376,8 @@ GrowPlanHost build_rstep_plan(Sym sym, MPO const& mpo, BoundaryIndex const& R, M
 
 // ---- block form of the MPO-term sum ------------------------------------------------------------
 // small-tile lines: those with the most shares of their terms first, then by lanes per share (the
-// power of two >= rows * cols), neighbours staying together, with their terms copied in that order
+// power of two >= rows * cols), then by term count (longest first, so that the lanes of a wave run loops
+// of similar length), with their terms copied in that order
 template <class Pred>
 static void build_small_lines(SBlockTable& B, HostTable<SLine> const& lines, HostTable<STerm> const& terms,
                               Pred is_small) {
@@ -1394,7 +1395,7 @@ static void build_small_lines(SBlockTable& B, HostTable<SLine> const& lines, Hos
         keys.push_back(Key{lg, ts, nt, i});
     }
     std::stable_sort(keys.begin(), keys.end(), [](Key const& a, Key const& b) {
-        return a.ts != b.ts ? a.ts > b.ts : a.lg < b.lg;
+        return a.ts != b.ts ? a.ts > b.ts : a.lg != b.lg ? a.lg < b.lg : a.nt > b.nt;
     });
     std::vector<int64_t> t_start(keys.size() + 1, 0);
     for (size_t q = 0; q < keys.size(); ++q) t_start[q + 1] = t_start[q] + keys[q].nt;

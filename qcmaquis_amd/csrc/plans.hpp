@@ -277,9 +277,9 @@ SBlockTable build_sblocks(HostTable<SLine> const& lines, HostTable<STerm> const&
 // those of the lines count), else 0.  Term by term every term fetches its tile; a block reads it once
 // for 64 lines, but each has its chain of tables, tiles and matrix cores, some 30 us with few blocks.
 // FP64 term sum in us, term by term / in blocks: 8 orbitals and M = 40 (0.2 million terms) 10.5 / 29, 9
-// and 60 (0.35) 23 / 40, 12 and 96 (2.2) 101 / 59, 18 and 128 (21) 488 / 253.  The line is on the safe
+// and 60 (0.35) 23 / 40, 12 and 96 (2.2) 97 / 59, 18 and 128 (21) 482 / 253.  The line is on the safe
 // side for the blocks: between 0.4 and 5 million terms those win where some tiles have more than 64
-// elements and go to blocks anyway (10 and M = 70, 0.76 million, 68 / 45; 11 and 80, 1.2, 95 / 66), and
+// elements and go to blocks anyway (10 and M = 70, 0.76 million, 68 / 45; 11 and 80, 1.2, 94 / 66), and
 // the terms where none has (10 and M = 45 23 / 39; 12 and 60, 2.2, 34 / 46; 14 and 50, 5.3, 38 / 54).
 // n_terms are those of all problems of a batch, so one of them may be summed in the other form, and
 // rounded otherwise, than in a plan of its own
