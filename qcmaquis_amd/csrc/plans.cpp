@@ -1394,9 +1394,15 @@ static void build_small_lines(SBlockTable& B, HostTable<SLine> const& lines, Hos
         while ((1 << (lg + ts)) < SMALL_LINE_LANES && nt > (SMALL_LINE_DEPTH << ts)) ++ts;
         keys.push_back(Key{lg, ts, nt, i});
     }
-    std::stable_sort(keys.begin(), keys.end(), [](Key const& a, Key const& b) {
-        return a.ts != b.ts ? a.ts > b.ts : a.lg != b.lg ? a.lg < b.lg : a.nt > b.nt;
-    });
+    // a counting pass: a comparison sort of some 40,000 lines would cost a quarter of the tables' time
+    constexpr int32_t KINDS = 9, NT = 1024;  // lanes and shares up to 2^8, term counts above told apart no more
+    auto rank = [](Key const& a) { return ((KINDS - 1 - a.ts) * KINDS + a.lg) * NT + NT - 1 - std::min(a.nt, NT - 1); };
+    std::vector<uint32_t> at(KINDS * KINDS * NT + 1, 0);
+    for (Key const& a : keys) ++at[size_t(rank(a)) + 1];
+    for (size_t r = 1; r < at.size(); ++r) at[r] += at[r - 1];
+    std::vector<Key> sorted(keys.size());
+    for (Key const& a : keys) sorted[at[size_t(rank(a))]++] = a;
+    keys.swap(sorted);
     std::vector<int64_t> t_start(keys.size() + 1, 0);
     for (size_t q = 0; q < keys.size(); ++q) t_start[q + 1] = t_start[q] + keys[q].nt;
     require(t_start.back() < int64_t(INT32_MAX), "S blocks: more than 2^31 small-tile terms");
@@ -1748,10 +1754,11 @@ void check_sblocks(SBlockTable const& B, uint64_t t_size, uint64_t s_size) {
             if (c) bad = std::max(bad, 4);
             c = 1;
         };
-        for (SWork const& w : B.work) mark(w, seen);
         const int64_t nt = B.n_work.team, np = B.n_work.pair, n = int64_t(B.work.size());
-        // an item of fewer waves than its tile needs would leave elements unwritten
         for (int64_t i = 0; bad == 0 && i < n; ++i) {
+            mark(B.work[size_t(i)], seen);
+            if (bad) break;
+            // an item of fewer waves than its tile needs would leave elements unwritten
             const int32_t E = B.blocks[size_t(B.work[size_t(i)].blk)].E;
             if (i < nt ? E <= 64 : i < nt + np ? E <= 32 || E > 64 : E > 32) bad = 4;
         }

@@ -118,13 +118,13 @@ uint64_t run_lines(HostTable<SLine>& lines, HostTable<STerm> const& terms, const
             ++small_covered;
         }
     for (char d : sdone) require(d, "emulated small lines: line not written");
-    // the lanes of a wave run loops of similar length: lines of one kind by term count
+    // the lanes of a wave run loops of similar length: lines of one kind by term count (up to 1023)
     for (size_t i = 0; i < B.small_work.size(); ++i)
         for (int32_t q = B.small_work[i].line0; q < B.small_work[i].line0 + B.small_work[i].n; ++q) {
             SSmallWork const& w = B.small_work[i];
             if (q == w.line0 && (i == 0 || B.small_work[i - 1].lg != w.lg || B.small_work[i - 1].ts != w.ts)) continue;
             SLine const &a = B.small_lines[size_t(q - 1)], &b = B.small_lines[size_t(q)];
-            require(a.t1 - a.t0 >= b.t1 - b.t0, "emulated small lines: not by term count");
+            require(a.t1 - a.t0 >= std::min(b.t1 - b.t0, 1023), "emulated small lines: not by term count");
         }
     std::vector<std::vector<char>> done(B.blocks.size());
     for (size_t i = 0; i < B.blocks.size(); ++i) done[i].assign(size_t(B.blocks[i].E) * SBLOCK_LINES, 0);
