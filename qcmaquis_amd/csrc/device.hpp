@@ -78,7 +78,7 @@ hipError_t launch_dots(VecPairs const& v, int count, uint64_t n, double* work, d
 // DOT_BLOCKS partials)
 hipError_t launch_gram_schmidt(double* t, const double* const* v, int count, uint64_t n, double* work, double* out,
                                hipStream_t stream);
-// out = sum of c[j] p[j], j < count, in order (count >= 1); out may be one of the operands
+// out = sum of c[j] p[j], j < count, in order (count >= 1); out may be one of the first VEC_MAX operands
 hipError_t launch_lincomb(double* out, const double* const* p, const double* c, int count, uint64_t n, hipStream_t stream);
 // y += coef * x with coef = sign * num[0] / (den ? den[0] : 1)  (coefficients stay on the device)
 hipError_t launch_axpy_dev(double* y, const double* x, uint64_t n, const double* num, const double* den, double sign,

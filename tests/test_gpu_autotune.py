@@ -1,5 +1,5 @@
-"""GEMM tile autotuner (MQ_OPT_AUTOTUNE) on the device: plans whose GEMM stages are scheduled by
-the timed pick of the candidate tile rules give the oracle's H*psi (1e-12 relative) at every site of
+"""GEMM autotuner (MQ_OPT_AUTOTUNE) on the device: plans whose GEMM stages are scheduled by
+the timed pick of the candidate splits along K give the oracle's H*psi (1e-12 relative) at every site of
 a chain with sectors above 64 states; every stage key is recorded once with a pick among the
 candidates, and a second plan of the same site problem takes the recorded picks without timing."""
 import numpy as np
