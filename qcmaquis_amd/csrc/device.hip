@@ -516,8 +516,8 @@ __global__ __launch_bounds__(SB_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
     // Non-finite elements of T: a zero coefficient times one is NaN in every line of its group, also in those
     // that do not read the tile.  Where a sum came out non-finite in the tiles that the term-by-term
     // sum may take instead (at most 64 elements), the lines are summed again over the tiles they read.  A
-    // non-finite element shows in every row of its group, so the first row is looked at: no cost beside
-    // the sum (18 orbitals, M = 128: 253 us with and without).
+    // non-finite element shows in every row of its group, so the first row is looked at: at 18 orbitals and
+    // M = 128, where all blocks are of such tiles, H*psi takes 324 us with the look and 322 without.
     if (!team) {
         bool odd = false;
 #pragma unroll
